@@ -8,16 +8,40 @@ namespace chimera {
 
 // One butterfly stage with stride h < 64 across the lanes of a wave: the
 // lower element of each pair becomes a + b and the upper a - b (FFHT runs
-// stages 1, 2, 4, ... in that order).
-__device__ __forceinline__ float butterfly_lanes(float x, int h, int l) {
-    const float p = __shfl_xor(x, h, kWave);
-    return (l & h) ? (p - x) : (x + p);
+// stages 1, 2, 4, ... in that order), each as its partner's value plus or
+// minus its own. The exchanges run on the vector ALU (DPP within a row of 16
+// lanes, the lane swaps past it), except h = 4, which no DPP pattern gives.
+template <int kH>
+__device__ __forceinline__ float butterfly_lanes(float x, int l) {
+    const uint32_t bits = __float_as_uint(x);
+    if constexpr (kH == 16 || kH == 32) {
+        // the swap leaves the lower lane's value in [0] and the upper lane's in [1]
+        const auto r = kH == 16 ? __builtin_amdgcn_permlane16_swap(bits, bits, false, false)
+                                : __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+        const float lo = __uint_as_float(r[0]), hi = __uint_as_float(r[1]);
+        return (l & kH) ? lo - hi : lo + hi;
+    } else {
+        int p;
+        if constexpr (kH == 1)
+            p = __builtin_amdgcn_mov_dpp(static_cast<int>(bits), 0xB1, 0xF, 0xF, true);  // quad_perm 1 0 3 2
+        else if constexpr (kH == 2)
+            p = __builtin_amdgcn_mov_dpp(static_cast<int>(bits), 0x4E, 0xF, 0xF, true);  // quad_perm 2 3 0 1
+        else if constexpr (kH == 4)
+            p = __builtin_amdgcn_ds_swizzle(static_cast<int>(bits), 0x101F);             // lane ^ 4
+        else
+            p = __builtin_amdgcn_mov_dpp(static_cast<int>(bits), 0x128, 0xF, 0xF, true);  // row_ror:8
+        const float s = (l & kH) ? -x : x;
+        return __int_as_float(p) + s;
+    }
 }
 
 __device__ __forceinline__ float fwht64_lanes(float x, int l) {
-#pragma unroll
-    for (int h = 1; h < 64; h <<= 1) x = butterfly_lanes(x, h, l);
-    return x;
+    x = butterfly_lanes<1>(x, l);
+    x = butterfly_lanes<2>(x, l);
+    x = butterfly_lanes<4>(x, l);
+    x = butterfly_lanes<8>(x, l);
+    x = butterfly_lanes<16>(x, l);
+    return butterfly_lanes<32>(x, l);
 }
 
 // Element j changes sign when bit j % 8 of byte j / 8 of the round's 16
