@@ -179,8 +179,11 @@ __global__ __launch_bounds__(256) void probe_centroids_kernel(const float* __res
 //         the conversion keeps (-0 for tiny misses). The rerank picks the
 //         hits out of the records.
 // MODE 2: minimum d' over the sampled tiles into ukey[row] (ordered key).
-// MODE 3: candidates {id, d' bits} with d' <= ukey[row] + 2 * probe_delta of
-//         the row into buf[L * lane_cap ...], their number into cnt[L].
+// MODE 3: candidates {id, d' bits} with d' <= b + 2 * probe_delta of the row
+//         into buf[L * lane_cap ...], their number into cnt[L]; b is the
+//         least d' the lane knows, ukey[row] (the sampled tiles') to start
+//         with. The exact nearest centroid c has d'(c) <= d(c) + delta <=
+//         d(x) + delta <= d'(x) + 2 delta for every x, so it is among them.
 //
 // Staging: the tiles of a stage go from global memory straight into LDS
 // (global_load_lds_dwordx4, no registers on the way), into one of two
@@ -234,6 +237,7 @@ __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
     bf16x8_t bq[kColBlocks][8];
     float th[kColBlocks];    // acc-space threshold -t/2: hit iff acc >= th
     float rmax[kColBlocks];  // MODE 2: max acc = -(min d')/2
+    float dl[kColBlocks];    // MODE 3: probe_delta of the row
     int lcnt[kColBlocks];
     float gmax[kColBlocks][kGroupsPerStage];
     size_t sub[kColBlocks];  // first entry of the lane's sub-list
@@ -267,7 +271,8 @@ __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
             // the two lane halves hold the two halves of the row
             const float qn = sqrtf(ss + __shfl_xor(ss, 32, kWave));
             const float eq = sqrtf(es + __shfl_xor(es, 32, kWave));
-            th[cb] = ok ? -0.5f * (ordered_to_float(ukey[row]) + 2.0f * probe_delta(qn, eq, cmax, ecmax)) : INFINITY;
+            dl[cb] = probe_delta(qn, eq, cmax, ecmax);
+            th[cb] = ok ? -0.5f * (ordered_to_float(ukey[row]) + 2.0f * dl[cb]) : INFINITY;
         } else {
             th[cb] = INFINITY;
         }
@@ -351,6 +356,8 @@ __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
                 }
                 lcnt[cb] += hit ? 1 : 0;
             } else if (m >= th[cb]) {  // MODE 3; th is +inf past the last row
+                // the lane's best so far bounds the nearest d' too
+                th[cb] = fmaxf(th[cb], m - dl[cb]);
                 // four values at a time, then one at a time: the wave
                 // skips what no lane hits, so a rare hit costs a
                 // compare per group of four and per value of one group
@@ -1071,55 +1078,116 @@ __global__ __launch_bounds__(kRerankWaves * kWave) void probe_rerank_kernel(
 }
 
 // Nearest centroid of each row among its buffered candidates by the exact
-// fp32 score (sequential fmaf dot, ties to the lower id). One wave per row;
-// rows with no candidate or a flag are left to the exact kernel.
+// fp32 score (sequential fmaf dot, ties to the lower id). Rows with no
+// candidate or a flag are left to the exact kernel.
+//
+// 16 lanes per row: the row's sub-lists hold the candidates of running
+// bounds (a handful), of which only those within 2 delta of the row's least
+// d' can be the nearest. Where one is left it is the label; the others are
+// scored in fp32, a lane each. What bounds it is the latency of those loads:
+// 1M rows over 4,096 centroids took 4.05 ms with one wave per row that
+// scored every buffered candidate and takes 0.48 ms (the filtered pass, with running bounds, 1.86 -> 1.35 ms).
+constexpr int kTop1Lanes = 16;
 __global__ __launch_bounds__(256) void probe_top1_rerank_kernel(const float* __restrict__ rows, int nrows,
                                                                 const float* __restrict__ centroids,
                                                                 const float* __restrict__ norms,
                                                                 const uint2* __restrict__ buf,
                                                                 const uint32_t* __restrict__ cnt, int lane_cap,
-                                                                int nsub, uint32_t* __restrict__ row_flag,
+                                                                int nsub, float cmax, float ecmax,
+                                                                uint32_t* __restrict__ row_flag,
                                                                 uint32_t* __restrict__ labels) {
-    const int row = blockIdx.x * 4 + wave_id();
-    const int l = lane_id();
-    if (row >= nrows) return;
-    if (row_flag[row]) return;
-    const float4* q = reinterpret_cast<const float4*>(rows + static_cast<size_t>(row) * kDim);
-    uint64_t best = ~0ull;
-    uint32_t total = 0;
-    for (int sb = 0; sb < nsub; ++sb) {
-        const uint32_t n = cnt[static_cast<size_t>(row) * nsub + sb];
-        total += n;
-        const uint2* src = buf + (static_cast<size_t>(row) * nsub + sb) * lane_cap;
-        for (uint32_t t = l; t < n; t += kWave) {
-            const uint32_t c = src[t].x;
-            const float4* cv = reinterpret_cast<const float4*>(centroids + static_cast<size_t>(c) * kDim);
-            float dot = 0.0f;
-            for (int j4 = 0; j4 < kDim / 4; ++j4) {
-                const float4 a = q[j4];
-                const float4 v = cv[j4];
-                dot = __fmaf_rn(a.x, v.x, dot);
-                dot = __fmaf_rn(a.y, v.y, dot);
-                dot = __fmaf_rn(a.z, v.z, dot);
-                dot = __fmaf_rn(a.w, v.w, dot);
-            }
-            const float score = norms[c] - 2.0f * dot;
-            const uint64_t key = (static_cast<uint64_t>(float_to_ordered(score)) << 32) | c;
-            best = key < best ? key : best;
+    const int row = static_cast<int>(blockIdx.x) * (256 / kTop1Lanes) + static_cast<int>(threadIdx.x) / kTop1Lanes;
+    const int j = static_cast<int>(threadIdx.x) % kTop1Lanes;
+    const bool live = row < nrows && row_flag[row < nrows ? row : 0] == 0u;
+    const size_t r = static_cast<size_t>(live ? row : 0);
+    const float4* q = reinterpret_cast<const float4*>(rows + r * kDim);
+    // |q| and |q - bf16(q)| for the margin
+    float ss = 0.0f, es = 0.0f;
+#pragma unroll
+    for (int u = 0; u < kDim / 4 / kTop1Lanes; ++u) {
+        const float4 v = q[u * kTop1Lanes + j];
+        const float x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float e = x[c] - bf16_round(x[c]);
+            ss = __fmaf_rn(x[c], x[c], ss);
+            es = __fmaf_rn(e, e, es);
         }
     }
-    if (total == 0) {
-        if (l == 0) row_flag[row] = 1u;
+#pragma unroll
+    for (int o = kTop1Lanes / 2; o >= 1; o >>= 1) {
+        ss += __shfl_xor(ss, o, kWave);
+        es += __shfl_xor(es, o, kWave);
+    }
+    const float delta = probe_delta(sqrtf(ss), sqrtf(es), cmax, ecmax);
+    // lane j walks sub-lists j % per, j % per + per, ... from entry j / per on
+    int per = 1;
+    while (per < nsub && per < kTop1Lanes) per *= 2;
+    const int step = kTop1Lanes / per;
+    auto walk = [&](auto&& visit) {
+        for (int sb = j & (per - 1); sb < nsub; sb += per) {
+            const uint32_t n = live ? cnt[r * nsub + sb] : 0u;
+            const uint2* src = buf + (r * nsub + sb) * lane_cap;
+            for (uint32_t t = static_cast<uint32_t>(j / per); t < n; t += step) visit(src[t]);
+        }
+    };
+    // the row's least d' and its number of candidates
+    float least = INFINITY;
+    int total = 0;
+    walk([&](const uint2& c) {
+        least = fminf(least, __uint_as_float(c.y));
+        ++total;
+    });
+#pragma unroll
+    for (int o = kTop1Lanes / 2; o >= 1; o >>= 1) {
+        least = fminf(least, __shfl_xor(least, o, kWave));
+        total += __shfl_xor(total, o, kWave);
+    }
+    if (live && total == 0 && j == 0) row_flag[row] = 1u;
+    // those that can be the nearest (all, should the bound not be a number)
+    const float reach = least + 2.0f * delta;
+    int left = 0;
+    uint32_t id = 0u;
+    walk([&](const uint2& c) {
+        if (!(__uint_as_float(c.y) > reach)) {
+            ++left;
+            id = c.x;
+        }
+    });
+    int all = left;
+#pragma unroll
+    for (int o = kTop1Lanes / 2; o >= 1; o >>= 1) all += __shfl_xor(all, o, kWave);
+    if (all == 1) {
+        if (left == 1) labels[row] = id;
         return;
     }
+    uint64_t best = ~0ull;
+    walk([&](const uint2& cd) {
+        if (__uint_as_float(cd.y) > reach) return;
+        const uint32_t c = cd.x;
+        const float4* cv = reinterpret_cast<const float4*>(centroids + static_cast<size_t>(c) * kDim);
+        float dot = 0.0f;
+#pragma unroll 8
+        for (int j4 = 0; j4 < kDim / 4; ++j4) {
+            const float4 a = q[j4];
+            const float4 v = cv[j4];
+            dot = __fmaf_rn(a.x, v.x, dot);
+            dot = __fmaf_rn(a.y, v.y, dot);
+            dot = __fmaf_rn(a.z, v.z, dot);
+            dot = __fmaf_rn(a.w, v.w, dot);
+        }
+        const float score = norms[c] - 2.0f * dot;
+        const uint64_t key = (static_cast<uint64_t>(float_to_ordered(score)) << 32) | c;
+        best = key < best ? key : best;
+    });
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
+    for (int m = kTop1Lanes / 2; m >= 1; m >>= 1) {
         const uint32_t lo = __shfl_xor(static_cast<uint32_t>(best), m, kWave);
         const uint32_t hi = __shfl_xor(static_cast<uint32_t>(best >> 32), m, kWave);
         const uint64_t o = (static_cast<uint64_t>(hi) << 32) | lo;
         best = o < best ? o : best;
     }
-    if (l == 0) labels[row] = static_cast<uint32_t>(best & 0xFFFFFFFFu);
+    if (live && total != 0 && j == 0) labels[row] = static_cast<uint32_t>(best & 0xFFFFFFFFu);
 }
 
 // ---- launchers ----
@@ -1305,8 +1373,9 @@ hipError_t launch_assign_top1(hipStream_t s, const ProbePlan& p, const float* ro
                        p.tiles_per_split, 1, nullptr, nullptr, buf, nullptr, nullptr, cnt, p.lane_cap, row_flag, ukey,
                        cmax, ecmax, p.row_blocks, p.splits);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(probe_top1_rerank_kernel, dim3((nrows + 3) / 4), dim3(256), 0, s, rows, nrows, centroids, norms,
-                       buf, cnt, p.lane_cap, 2 * p.splits, row_flag, labels);
+    constexpr int kTop1Rows = 256 / kTop1Lanes;
+    hipLaunchKernelGGL(probe_top1_rerank_kernel, dim3((nrows + kTop1Rows - 1) / kTop1Rows), dim3(256), 0, s, rows, nrows,
+                       centroids, norms, buf, cnt, p.lane_cap, 2 * p.splits, cmax, ecmax, row_flag, labels);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     return launch_probe_exact_flagged(s, rows, nrows, centroids, norms, k, 1, row_flag, labels, fb);
 }
