@@ -937,7 +937,7 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
     // IVF lists and the cluster-ordered arrays (ivf_pg.cpp:110-126,
     // build_index.cu:328-363)
     {
-        uint32_t *keys_out = nullptr, *vals_in = nullptr, *token_doc_u = nullptr, *runs_d = nullptr;
+        uint32_t *keys_out = nullptr, *vals_in = nullptr, *token_doc_u = nullptr;
         CK(tmp.alloc(&keys_out, n, "sorted assignments"));
         CK(tmp.alloc(&vals_in, n, "token ids"));
         CK(dev_alloc(c, c->index_allocs, &c->inv, n, "IVF lists"));
@@ -955,10 +955,9 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
         CK(dev_alloc(c, c->index_allocs, &c->f1_clu, n, "clustered factors"));
         CK(dev_alloc(c, c->index_allocs, &c->doc_clu, n, "clustered doc ids"));
         CK(tmp.alloc(&token_doc_u, n, "token documents"));
-        CK(tmp.alloc(&runs_d, K, "cluster runs"));
         CK_HIP(launch_layout(s, keys_out, c->inv, c->n, c->n_clusters, c->doc_ptrs, c->num_docs, c->codes_tok,
                              c->f1_tok, reinterpret_cast<int32_t*>(token_doc_u), c->cluster_pos, c->codes_clu,
-                             c->f1_clu, c->doc_clu, runs_d),
+                             c->f1_clu, c->doc_clu),
                "index layout");
     }
     uint32_t st = 0;

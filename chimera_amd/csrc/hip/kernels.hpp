@@ -189,7 +189,7 @@ hipError_t launch_sort_assignments(hipStream_t s, const uint32_t* labels, int64_
 hipError_t launch_layout(hipStream_t s, const uint32_t* sorted_keys, const uint32_t* inv, int64_t n, int64_t k,
                          const int32_t* doc_ptrs, int64_t m, const uint8_t* codes_tok, const float* f1_tok,
                          int32_t* token_doc, uint64_t* cluster_pos, uint8_t* codes_clu, float* f1_clu,
-                         int32_t* doc_clu, uint32_t* runs);
+                         int32_t* doc_clu);
 
 // Token-order copies of the clustered one-bit data: out[t] = in[pos[t]].
 hipError_t launch_gather_token_order(hipStream_t s, const uint8_t* codes_clu, const float* f1_clu,

@@ -1,6 +1,6 @@
 // Index build on the GPU (build_index.cu:258-363, quantization.cpp:32-193,
 // ivf_pg.cpp:110-126): rotation and one-bit / full-code encoding of every
-// token, the cluster-ordered layout and the per-cluster document runs.
+// token and the cluster-ordered layout.
 // The arithmetic mirrors the host encoder operation for operation (the same
 // fused multiply-adds, the same sequential sums, the same event order in
 // best_rescale_factor) so both builds produce identical bytes.
@@ -655,17 +655,6 @@ __global__ void reorder_kernel(const uint32_t* __restrict__ inv, int64_t n, cons
     doc_clu[p] = token_doc[t];
 }
 
-// Number of runs of equal document ids inside each cluster.
-__global__ void cluster_runs_kernel(const uint64_t* __restrict__ cluster_pos, const int32_t* __restrict__ doc_clu,
-                                    int64_t k, uint32_t* __restrict__ runs) {
-    const int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (c >= k) return;
-    uint32_t r = 0;
-    for (uint64_t p = cluster_pos[c]; p < cluster_pos[c + 1]; ++p)
-        if (p == cluster_pos[c] || doc_clu[p] != doc_clu[p - 1]) ++r;
-    runs[c] = r;
-}
-
 // ---- launchers ----
 
 namespace {
@@ -712,7 +701,7 @@ hipError_t launch_sort_assignments(hipStream_t s, const uint32_t* labels, int64_
 hipError_t launch_layout(hipStream_t s, const uint32_t* sorted_keys, const uint32_t* inv, int64_t n, int64_t k,
                          const int32_t* doc_ptrs, int64_t m, const uint8_t* codes_tok, const float* f1_tok,
                          int32_t* token_doc, uint64_t* cluster_pos, uint8_t* codes_clu, float* f1_clu,
-                         int32_t* doc_clu, uint32_t* runs) {
+                         int32_t* doc_clu) {
     hipLaunchKernelGGL(cluster_bounds_kernel, dim3(blocks_for(k + 1, 256)), dim3(256), 0, s, sorted_keys, n, k,
                        cluster_pos);
     hipError_t e = hipGetLastError();
@@ -721,8 +710,6 @@ hipError_t launch_layout(hipStream_t s, const uint32_t* sorted_keys, const uint3
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(reorder_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, s, inv, n, codes_tok, f1_tok, token_doc,
                        codes_clu, f1_clu, doc_clu);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(cluster_runs_kernel, dim3(blocks_for(k, 256)), dim3(256), 0, s, cluster_pos, doc_clu, k, runs);
     return hipGetLastError();
 }
 

@@ -30,6 +30,7 @@
 // -|c|^2/2, so acc = <q_b,c_b> - |c|^2/2 = -d'/2 and d' <= t is acc >= -t/2
 // (exact: scaling by powers of two): the per-tile test is a max over the
 // lane's 16 values and one compare, with no per-value arithmetic.
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -145,26 +146,35 @@ __device__ __forceinline__ __attribute__((address_space(3))) void* lds_ptr(void*
 
 // bf16 copies of the centroids, the probe's accumulator start -|c|^2/2 and
 // max over centroids of |c - c_b| (atomicMax on the bits of a non-negative
-// float into *err_max, which the caller clears). One wave per centroid.
+// float into *err_max, which the caller clears). One wave per centroid at a
+// time, one atomic per block: an atomic per centroid on the one word took
+// 0.38 ms for 32,768 centroids, this 0.02 ms.
+constexpr int kCentroidBlocks = 1024;
 __global__ __launch_bounds__(256) void probe_centroids_kernel(const float* __restrict__ c,
                                                               const float* __restrict__ norms, int64_t k,
                                                               uint16_t* __restrict__ out, float* __restrict__ nhalf,
                                                               uint32_t* __restrict__ err_max) {
-    const int64_t cen = static_cast<int64_t>(blockIdx.x) * (blockDim.x / kWave) + wave_id();
-    if (cen >= k) return;
+    __shared__ uint32_t most;
+    if (threadIdx.x == 0) most = 0u;
+    __syncthreads();
     const int l = lane_id();
-    const float2 v = reinterpret_cast<const float2*>(c + cen * kDim)[l];
-    const uint16_t hx = f32_to_bf16_rne(v.x), hy = f32_to_bf16_rne(v.y);
-    reinterpret_cast<uint32_t*>(out + cen * kDim)[l] = static_cast<uint32_t>(hx) | (static_cast<uint32_t>(hy) << 16);
-    const float ex = v.x - __uint_as_float(static_cast<uint32_t>(hx) << 16);
-    const float ey = v.y - __uint_as_float(static_cast<uint32_t>(hy) << 16);
-    float es = ex * ex + ey * ey;
+    uint32_t own = 0u;
+    for (int64_t cen = static_cast<int64_t>(blockIdx.x) * 4 + wave_id(); cen < k; cen += static_cast<int64_t>(gridDim.x) * 4) {
+        const float2 v = reinterpret_cast<const float2*>(c + cen * kDim)[l];
+        const uint16_t hx = f32_to_bf16_rne(v.x), hy = f32_to_bf16_rne(v.y);
+        reinterpret_cast<uint32_t*>(out + cen * kDim)[l] = static_cast<uint32_t>(hx) | (static_cast<uint32_t>(hy) << 16);
+        const float ex = v.x - __uint_as_float(static_cast<uint32_t>(hx) << 16);
+        const float ey = v.y - __uint_as_float(static_cast<uint32_t>(hy) << 16);
+        float es = ex * ex + ey * ey;
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) es += __shfl_xor(es, o, kWave);
-    if (l == 0) {
-        nhalf[cen] = -0.5f * norms[cen];
-        atomicMax(err_max, __float_as_uint(sqrtf(es)));
+        for (int o = 32; o >= 1; o >>= 1) es += __shfl_xor(es, o, kWave);
+        const uint32_t e = __float_as_uint(sqrtf(es));
+        own = e > own ? e : own;
+        if (l == 0) nhalf[cen] = -0.5f * norms[cen];
     }
+    if (l == 0) atomicMax(&most, own);
+    __syncthreads();
+    if (threadIdx.x == 0 && most != 0u) atomicMax(err_max, most);
 }
 
 // MODE 0: minima of groups of G sampled tiles into gm[row][group]
@@ -1196,8 +1206,8 @@ hipError_t launch_probe_centroids(hipStream_t s, const float* c, const float* no
                                   float* nhalf, uint32_t* err_max) {
     hipError_t e = launch_fill_u32(s, err_max, 1, 0u);
     if (e != hipSuccess || k == 0) return e;
-    hipLaunchKernelGGL(probe_centroids_kernel, dim3(static_cast<unsigned>((k + 3) / 4)), dim3(256), 0, s, c, norms, k,
-                       cbf, nhalf, err_max);
+    hipLaunchKernelGGL(probe_centroids_kernel, dim3(static_cast<unsigned>(std::min<int64_t>((k + 3) / 4, kCentroidBlocks))),
+                       dim3(256), 0, s, c, norms, k, cbf, nhalf, err_max);
     return hipGetLastError();
 }
 
