@@ -255,13 +255,21 @@ __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
     for (int cb = 0; cb < kColBlocks; ++cb) {
         const int row = row0 + 32 * cb + j;
         const bool ok = row < nrows;
-        const float* src = rot + static_cast<size_t>(ok ? row : 0) * kDim;
+        // all of the lane's loads first (row 0 stands in past the end), then
+        // the conversions: a load per value under its own condition made the
+        // prologue a chain of round trips
+        const float4* src = reinterpret_cast<const float4*>(rot + static_cast<size_t>(ok ? row : 0) * kDim);
+        float4 raw[16];
+#pragma unroll
+        for (int s = 0; s < 16; ++s) raw[s] = src[4 * (s >> 1) + 2 * hk + (s & 1)];
         float ss = 0.0f, es = 0.0f;
 #pragma unroll
         for (int s = 0; s < 8; ++s)
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const float v = ok ? src[16 * s + 8 * hk + e] : 0.0f;
+                const float4 r4 = raw[2 * s + (e >> 2)];
+                const float x = (e & 3) == 0 ? r4.x : (e & 3) == 1 ? r4.y : (e & 3) == 2 ? r4.z : r4.w;
+                const float v = ok ? x : 0.0f;
                 const uint16_t h = f32_to_bf16_rne(v);
                 if (MODE == 3) {
                     const float ev = v - __uint_as_float(static_cast<uint32_t>(h) << 16);
