@@ -190,6 +190,7 @@ struct chimera_ctx {
     uint32_t* w_out_status = nullptr;
     size_t w_out_used = 0;             // bytes of the region the last call laid out
     unsigned char* h_stage = nullptr;  // pinned host memory (hipHostMalloc)
+    unsigned char* d_stage = nullptr;  // the same memory as the device sees it
     size_t h_stage_bytes = 0;
     uint32_t* noalloc_status = nullptr;  // status word of the last chimera_search_device_noalloc (own allocation)
     bool noalloc_pending = false;        // that word has not been read by chimera_synchronize
@@ -559,7 +560,7 @@ int run_candidates(chimera_ctx* c, const Workspace& w, hipStream_t s, int qb, in
 }
 
 // Rotation, LUT and probe of queries [qb, qb + nq) (d_queries is the whole
-// batch). The matrix-core probe runs at every batch size (one query at docs2m:
+// batch); the rotation clears the batch's status word. The matrix-core probe runs at every batch size (one query at docs2m:
 // 0.19 ms against 52 ms for the exact vector kernel, whose 8-row blocks leave
 // the GPU idle); its buffers belong to the context, allocated at upload.
 int run_front(chimera_ctx* c, const Workspace& w, hipStream_t s, const float* d_queries, int32_t qb, int32_t nq) {
@@ -568,7 +569,7 @@ int run_front(chimera_ctx* c, const Workspace& w, hipStream_t s, const float* d_
     uint32_t* labels = w.labels + q0 * kQ * static_cast<size_t>(c->opt.nprobe);
     STAGE(c, 0, launch_rotate_lut(s, d_queries + q0 * kQ * static_cast<size_t>(c->dim), nq, static_cast<int>(c->dim),
                                   c->flips, static_cast<int>(c->ex_bits), rot, w.cb1 + q0 * kQ,
-                                  w.cbex + q0 * kQ, w.lut + q0 * kLutPerQuery),
+                                  w.cbex + q0 * kQ, w.lut + q0 * kLutPerQuery, w.err),
           "rotation kernel");
     const int nrows = nq * kQ;
     const ProbePlan plan = plan_probe_mfma(nrows, c->n_clusters, c->opt.nprobe, c->num_cus);
@@ -591,8 +592,9 @@ int run_front(chimera_ctx* c, const Workspace& w, hipStream_t s, const float* d_
 
 // One-bit refine, chunked selection, full-bit scoring and top-k of queries
 // [qb, qb + nq); d_ids / d_scores / d_counts are the whole batch's outputs.
+// d_status, if given, receives the status word.
 int run_back(chimera_ctx* c, const Workspace& w, hipStream_t s, int32_t qb, int32_t nq, int32_t k, int64_t* d_ids,
-             float* d_scores, int32_t* d_counts) {
+             float* d_scores, int32_t* d_counts, uint32_t* d_status) {
     const chimera_search_options& o = c->opt;
     const size_t q0 = static_cast<size_t>(qb);
     const size_t kr = static_cast<size_t>(o.k_refine), fb = static_cast<size_t>(c->fb_cap);
@@ -627,25 +629,32 @@ int run_back(chimera_ctx* c, const Workspace& w, hipStream_t s, int32_t qb, int3
               "full-bit kernel");
     }
     STAGE(c, 12, launch_final_topk(s, nq, fcount, fids, fscores, c->fb_cap, k, d_ids + q0 * static_cast<size_t>(k),
-                                   d_scores ? d_scores + q0 * static_cast<size_t>(k) : nullptr, d_counts + q0),
+                                   d_scores ? d_scores + q0 * static_cast<size_t>(k) : nullptr, d_counts + q0, w.err,
+                                   d_status),
           "top-k kernel");
     return CHIMERA_OK;
 }
 
 int run_pipeline(chimera_ctx* c, const Workspace& w, const float* d_queries, int32_t nq, int32_t k, int64_t* d_ids,
-                 float* d_scores, int32_t* d_counts) {
+                 float* d_scores, int32_t* d_counts, uint32_t* d_status = nullptr) {
     if (nq == 0) return CHIMERA_OK;
     hipStream_t s = c->stream;
-    CK_HIP(launch_fill_u32(s, w.err, 1, 0u), "clearing status");
     CK(run_front(c, w, s, d_queries, 0, nq));
     CK(run_candidates(c, w, s, 0, nq));
-    return run_back(c, w, s, 0, nq, k, d_ids, d_scores, d_counts);
+    return run_back(c, w, s, 0, nq, k, d_ids, d_scores, d_counts, d_status);
 }
+
+// Host batches of up to this many bytes of queries (eight of 128 dimensions)
+// skip the copies, each a launch of its own around a search of a few
+// hundred us. 37 queries (0.45 MB) took the same either way (541 and 545 us):
+// there the read over PCIe costs what the copy does.
+constexpr size_t kDirectBytes = size_t{1} << 17;
 
 // Lays out the result region of a host call of nq queries and k results
 // (growing it, and the pinned staging buffer to hold it or host_bytes of
-// input, when needed).
-int ensure_out(chimera_ctx* c, int32_t nq, int32_t k, size_t host_bytes) {
+// input, when needed): in the staging buffer itself with `direct` and a
+// staging buffer that the device can address, else in device memory.
+int ensure_out(chimera_ctx* c, int32_t nq, int32_t k, size_t host_bytes, bool direct = false) {
     const size_t m = static_cast<size_t>(nq) * static_cast<size_t>(k);
     const size_t used = m * 12 + static_cast<size_t>(nq) * 4 + 4;
     if (used > c->w_out_bytes) {
@@ -668,17 +677,21 @@ int ensure_out(chimera_ctx* c, int32_t nq, int32_t k, size_t host_bytes) {
         CK_HIP(hipStreamSynchronize(c->stream), "synchronising before staging growth");
         if (c->h_stage) (void)hipHostFree(c->h_stage);
         c->h_stage = nullptr;
+        c->d_stage = nullptr;
         c->h_stage_bytes = 0;
         const size_t bytes = (host + 4095) / 4096 * 4096;
         void* p = nullptr;
         CK_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault), "pinned staging buffer");
         c->h_stage = static_cast<unsigned char*>(p);
         c->h_stage_bytes = bytes;
+        void* dp = nullptr;
+        c->d_stage = hipHostGetDevicePointer(&dp, p, 0) == hipSuccess ? static_cast<unsigned char*>(dp) : nullptr;
     }
-    c->w_out_ids = reinterpret_cast<int64_t*>(c->w_out);
-    c->w_out_scores = reinterpret_cast<float*>(c->w_out + m * 8);
-    c->w_out_counts = reinterpret_cast<int32_t*>(c->w_out + m * 12);
-    c->w_out_status = reinterpret_cast<uint32_t*>(c->w_out + m * 12 + static_cast<size_t>(nq) * 4);
+    unsigned char* base = direct && c->d_stage ? c->d_stage : c->w_out;
+    c->w_out_ids = reinterpret_cast<int64_t*>(base);
+    c->w_out_scores = reinterpret_cast<float*>(base + m * 8);
+    c->w_out_counts = reinterpret_cast<int32_t*>(base + m * 12);
+    c->w_out_status = reinterpret_cast<uint32_t*>(base + m * 12 + static_cast<size_t>(nq) * 4);
     c->w_out_used = used;
     return CHIMERA_OK;
 }
@@ -1179,14 +1192,11 @@ int chimera_search_device_noalloc(chimera_ctx* c, const float* d_queries, int32_
     int r = CHIMERA_OK;
     const hipError_t e = launch_fill_u32(c->stream, reinterpret_cast<uint32_t*>(w.rcount), nq, 0u);
     if (e != hipSuccess) r = fail(CHIMERA_ERR_HIP, std::string("clearing refined counts failed: ") + hipGetErrorString(e));
-    if (r == CHIMERA_OK) r = run_pipeline(c, w, d_queries, nq, k, d_out_ids, d_out_scores, d_out_counts);
     // the status word moves out of the shared array into the context's own
     // word, so a later call on another context cannot overwrite it before
     // chimera_synchronize reads it
-    if (r == CHIMERA_OK) {
-        const hipError_t ce = launch_copy_u32(c->stream, c->noalloc_status, w.err, 1);
-        if (ce != hipSuccess) r = fail(CHIMERA_ERR_HIP, std::string("status copy failed: ") + hipGetErrorString(ce));
-    }
+    if (r == CHIMERA_OK)
+        r = run_pipeline(c, w, d_queries, nq, k, d_out_ids, d_out_scores, d_out_counts, c->noalloc_status);
     c->profiling = prof;
     if (r == CHIMERA_OK) c->noalloc_pending = true;
     return r;
@@ -1211,14 +1221,23 @@ int chimera_search(chimera_ctx* c, const float* queries, int32_t nq, int32_t k, 
     if (!queries || !out_ids || !out_counts) return fail(CHIMERA_ERR_INVALID_ARGUMENT, "null argument");
     CK(set_device(c));
     const size_t qbytes = static_cast<size_t>(nq) * kQ * static_cast<size_t>(c->dim) * sizeof(float);
-    CK(ensure_out(c, nq, k, qbytes));
-    // the batch goes up, and the results and status word come back, through
-    // the pinned staging buffer: one DMA copy each way
+    // The batch goes up, and the results and status word come back, through
+    // the pinned staging buffer. Up to kDirectBytes of queries, the rotation
+    // reads them and the top-k writes its results there over PCIe (the first
+    // and the last kernel, each word once); larger batches take a DMA copy
+    // each way.
+    bool direct = qbytes <= kDirectBytes;
+    CK(ensure_out(c, nq, k, qbytes, direct));
+    direct = direct && c->d_stage;
     std::memcpy(c->h_stage, queries, qbytes);
-    CK_HIP(hipMemcpyAsync(c->ws.queries, c->h_stage, qbytes, hipMemcpyHostToDevice, c->stream), "query upload");
-    CK(run_pipeline(c, c->ws, c->ws.queries, nq, k, c->w_out_ids, c->w_out_scores, c->w_out_counts));
-    CK_HIP(launch_copy_u32(c->stream, c->w_out_status, c->ws.err, 1), "search status");
-    CK_HIP(hipMemcpyAsync(c->h_stage, c->w_out, c->w_out_used, hipMemcpyDeviceToHost, c->stream), "result copy");
+    const float* d_queries = c->ws.queries;
+    if (direct)
+        d_queries = reinterpret_cast<const float*>(c->d_stage);
+    else
+        CK_HIP(hipMemcpyAsync(c->ws.queries, c->h_stage, qbytes, hipMemcpyHostToDevice, c->stream), "query upload");
+    CK(run_pipeline(c, c->ws, d_queries, nq, k, c->w_out_ids, c->w_out_scores, c->w_out_counts, c->w_out_status));
+    if (!direct)
+        CK_HIP(hipMemcpyAsync(c->h_stage, c->w_out, c->w_out_used, hipMemcpyDeviceToHost, c->stream), "result copy");
     CK_HIP(hipStreamSynchronize(c->stream), "search");
     const size_t m = static_cast<size_t>(nq) * k;
     std::memcpy(out_ids, c->h_stage, m * sizeof(int64_t));
@@ -1240,7 +1259,6 @@ int chimera_search_trace(chimera_ctx* c, const float* queries, int32_t nq, int32
     CK(ensure_out(c, nq, k, 0));
     const Workspace& w = c->ws;
     CK_HIP(hipMemcpyAsync(w.queries, queries, qbytes, hipMemcpyHostToDevice, s), "query upload");
-    CK_HIP(launch_fill_u32(s, w.err, 1, 0u), "clearing status");
     CK(run_front(c, w, s, w.queries, 0, nq));
     const size_t NQ = static_cast<size_t>(nq);
     auto d2h = [&](void* dst, const void* src, size_t bytes) -> int {
@@ -1282,7 +1300,7 @@ int chimera_search_trace(chimera_ctx* c, const float* queries, int32_t nq, int32
         }
         CK_HIP(hipStreamSynchronize(s), "trace");
     }
-    CK(run_back(c, w, s, 0, nq, k, c->w_out_ids, c->w_out_scores, w.out_counts));
+    CK(run_back(c, w, s, 0, nq, k, c->w_out_ids, c->w_out_scores, w.out_counts, nullptr));
     const size_t kr = static_cast<size_t>(c->opt.k_refine);
     CK(d2h(tr->refined_count, w.rcount, NQ * 4));
     CK(d2h(tr->refined_ids, w.rids, NQ * kr * 4));
@@ -1444,7 +1462,7 @@ int chimera_rotate_lut_device(chimera_ctx* c, const float* d_queries, int32_t nq
     if (nq == 0) return CHIMERA_OK;
     CK(set_device(c));
     CK_HIP(launch_rotate_lut(c->stream, d_queries, nq, static_cast<int>(c->dim), c->flips,
-                             static_cast<int>(c->ex_bits), d_rotated, d_cb1, d_cbex, d_lut),
+                             static_cast<int>(c->ex_bits), d_rotated, d_cb1, d_cbex, d_lut, nullptr),
            "rotation kernel");
     return CHIMERA_OK;
 }

@@ -16,8 +16,9 @@ hipError_t configure_candidate_kernels(int nbk, int k_refine);
 hipError_t configure_score_kernels(int k_refine, int fb_cap);
 hipError_t configure_query_kernels(int nprobe);
 
+// status: a word cleared along (may be null).
 hipError_t launch_rotate_lut(hipStream_t s, const float* queries, int nq, int dim, const uint8_t* flips,
-                             int ex_bits, float* rot, float* cb1, float* cbex, float* lut);
+                             int ex_bits, float* rot, float* cb1, float* cbex, float* lut, uint32_t* status);
 hipError_t launch_centroid_norms(hipStream_t s, const float* c, int64_t k, float* norms);
 hipError_t launch_probe_exact(hipStream_t s, const float* rot, int nrows, const float* centroids,
                               const float* norms, int64_t k, int nprobe, uint32_t* labels);
@@ -87,10 +88,12 @@ hipError_t launch_assign_top1(hipStream_t s, const ProbePlan& p, const float* ro
                               float ecmax, uint32_t* ukey, uint2* buf, uint32_t* cnt, uint32_t* row_flag,
                               uint32_t* labels, const ExactFallback& fb);
 // Exact probe of the flagged rows: listed and split over the centroids (fb),
-// or by the row-block kernel when more than fb.list_cap rows are flagged.
+// or by row blocks when more than fb.list_cap rows are flagged. `listed`:
+// the caller has filled fb.list and fb.nflag, else they are made from
+// row_flag here.
 hipError_t launch_probe_exact_flagged(hipStream_t s, const float* rot, int nrows, const float* centroids,
                                       const float* norms, int64_t k, int nprobe, const uint32_t* row_flag,
-                                      uint32_t* labels, const ExactFallback& fb);
+                                      uint32_t* labels, const ExactFallback& fb, bool listed);
 hipError_t launch_unpack_codes(hipStream_t s, int width, const uint8_t* packed, int64_t n, uint8_t* raw);
 
 // Candidate stage (kernels_candidates.hip). Per sub-batch of qs queries:
@@ -171,9 +174,11 @@ constexpr int kFullbitPadTokens = 16;
 hipError_t launch_fullbit_mfma(hipStream_t s, int nq, const float* rot, const float* cbex, const int32_t* fcount,
                                const int32_t* fids, int fb_cap, const int32_t* doc_ptrs, const uint8_t* full_codes,
                                const float* full_factors, int width, float* fscores, int num_cus);
+// status, out_status: a word copied along when both are given (the batch's
+// status, beside the results).
 hipError_t launch_final_topk(hipStream_t s, int nq, const int32_t* fcount, const int32_t* fids,
                              const float* fscores, int fb_cap, int k, int64_t* out_ids, float* out_scores,
-                             int32_t* out_counts);
+                             int32_t* out_counts, const uint32_t* status = nullptr, uint32_t* out_status = nullptr);
 
 // Index build (kernels_build.hip).
 hipError_t launch_encode_tokens(hipStream_t s, const float* emb, int64_t n, int dim, const uint8_t* flips,

@@ -726,17 +726,23 @@ __global__ __launch_bounds__(kF32Waves * kWave) void probe_mfma_f32_kernel(
 // select over ordered keys staged in LDS; thr = U + 2*delta. One 256-thread
 // block per row; the row's minima are contiguous (gm[row][group]). delta
 // takes |q - bf16(q)| times eq_weight: 1 for bf16 query operands, 0 for
-// fp32 ones (with ecmax 0 too).
+// fp32 ones (with ecmax 0 too). The threshold kernels also clear the rows'
+// flags and the count of flagged rows for the passes that follow.
 __global__ __launch_bounds__(256) void probe_threshold_kernel(const float* __restrict__ gm, int n_sampled,
                                                               int nrows, int rank, const float* __restrict__ rot,
                                                               float cmax, float ecmax, float eq_weight,
-                                                              float* __restrict__ thr) {
+                                                              float* __restrict__ thr, uint32_t* __restrict__ row_flag,
+                                                              uint32_t* __restrict__ nflag) {
     extern __shared__ uint32_t skey[];  // [n_sampled]
     __shared__ __align__(16) int hist[256];
     __shared__ uint32_t s_prefix;
     __shared__ int s_rem;
     const int row = blockIdx.x;
     if (row >= nrows) return;
+    if (threadIdx.x == 0) {
+        row_flag[row] = 0u;
+        if (row == 0) *nflag = 0u;
+    }
     const float* src = gm + static_cast<size_t>(row) * n_sampled;
     for (int g = threadIdx.x; g < n_sampled; g += blockDim.x) skey[g] = float_to_ordered(src[g]);
     __syncthreads();
@@ -758,11 +764,17 @@ template <int kPerLane>
 __global__ __launch_bounds__(256) void probe_threshold_wave_kernel(const float* __restrict__ gm, int n_groups,
                                                                    int nrows, int rank, const float* __restrict__ rot,
                                                                    float cmax, float ecmax, float eq_weight,
-                                                                   float* __restrict__ thr) {
+                                                                   float* __restrict__ thr,
+                                                                   uint32_t* __restrict__ row_flag,
+                                                                   uint32_t* __restrict__ nflag) {
     __shared__ __align__(16) int hist_all[4][256];
     const int l = lane_id();
     const int row = static_cast<int>(blockIdx.x) * 4 + wave_id();
     if (row >= nrows) return;
+    if (l == 0) {
+        row_flag[row] = 0u;
+        if (row == 0) *nflag = 0u;
+    }
     int* hist = hist_all[wave_id()];
     const float* src = gm + static_cast<size_t>(row) * n_groups;
     uint32_t key[kPerLane];
@@ -837,7 +849,8 @@ __global__ __launch_bounds__(kRerankWaves * kWave) void probe_rerank_kernel(
     const float* __restrict__ rot, int nrows, const float* __restrict__ centroids, const float* __restrict__ norms,
     const uint4* __restrict__ rval, const uint32_t* __restrict__ rtile, const uint32_t* __restrict__ cnt,
     int lane_cap, int nsub, int max_n, int nprobe, bool rigorous, float cmax, float ecmax, float eq_weight,
-    uint32_t* __restrict__ row_flag, uint32_t* __restrict__ row_cand, uint32_t* __restrict__ labels) {
+    uint32_t* __restrict__ row_flag, uint32_t* __restrict__ row_cand, uint32_t* __restrict__ labels,
+    uint32_t* __restrict__ list, uint32_t* __restrict__ nflag, int list_cap) {
     extern __shared__ uint64_t smem_keys[];  // [kRerankWaves][max_n]
     __shared__ float qs[kRerankWaves][kDim];
     __shared__ __align__(16) int hist_all[kRerankWaves][256];
@@ -845,8 +858,16 @@ __global__ __launch_bounds__(kRerankWaves * kWave) void probe_rerank_kernel(
     const int l = lane_id();
     const int row = static_cast<int>(blockIdx.x) * kRerankWaves + w;
     if (row >= nrows) return;
-    if (row_flag[row]) {
-        if (l == 0) row_cand[row] = 0xFFFFFFFFu;  // a sub-list overflowed in the filtered pass
+    // a row for the exact kernels: flagged and listed, by lane 0
+    auto leave = [&](uint32_t why) {
+        if (l != 0) return;
+        row_cand[row] = why;
+        row_flag[row] = 1u;
+        const uint32_t f = atomicAdd(nflag, 1u);
+        if (f < static_cast<uint32_t>(list_cap)) list[f] = static_cast<uint32_t>(row);
+    };
+    if (row_flag[row]) {  // a sub-list overflowed in the filtered pass
+        leave(0xFFFFFFFFu);
         return;
     }
     uint64_t* keys = smem_keys + static_cast<size_t>(w) * max_n;
@@ -939,10 +960,7 @@ __global__ __launch_bounds__(kRerankWaves * kWave) void probe_rerank_kernel(
         hmax = x > hmax ? x : hmax;
     }
     if (n > max_n || n < nprobe || hmax >= 0x7BFFu) {
-        if (l == 0) {
-            row_cand[row] = n > max_n ? 0xFFFFFFFFu : 0xFFFFFFFEu;
-            row_flag[row] = 1u;
-        }
+        leave(n > max_n ? 0xFFFFFFFFu : 0xFFFFFFFEu);
         return;
     }
     wave_lds_sync();
@@ -1005,10 +1023,7 @@ __global__ __launch_bounds__(kRerankWaves * kWave) void probe_rerank_kernel(
     // construction, while the check, through v's fp16 rounding, could not
     // certify the one lying exactly at U)
     if (!rigorous && !(vstar >= add_up(delta, eta))) {
-        if (l == 0) {
-            row_cand[row] = 0xFFFFFFFEu;
-            row_flag[row] = 1u;
-        }
+        leave(0xFFFFFFFEu);
         return;
     }
     if (l == 0) row_cand[row] = static_cast<uint32_t>(n);
@@ -1285,7 +1300,6 @@ hipError_t launch_probe_mfma(hipStream_t s, const ProbePlan& p, const float* rot
     const float ec = f32 ? 0.0f : ecmax;
     const float eqw = f32 ? 0.0f : 1.0f;
     if (part < 0 || part == 0) {
-        if ((e = launch_fill_u32(s, row_flag, nrows, 0u)) != hipSuccess) return e;
         // pass A over sampled tiles: gm index = sampled tile number, so the
         // split grid walks sampled tiles in order
         if (f32) {
@@ -1310,16 +1324,16 @@ hipError_t launch_probe_mfma(hipStream_t s, const ProbePlan& p, const float* rot
         const dim3 wgrid((nrows + 3) / 4);
         if (n_groups <= 8 * kWave)
             hipLaunchKernelGGL(probe_threshold_wave_kernel<8>, wgrid, dim3(256), 0, s, gm, n_groups, nrows, p.u_rank,
-                               rot, cmax, ec, eqw, thr);
+                               rot, cmax, ec, eqw, thr, row_flag, fb.nflag);
         else if (n_groups <= 16 * kWave)
             hipLaunchKernelGGL(probe_threshold_wave_kernel<16>, wgrid, dim3(256), 0, s, gm, n_groups, nrows,
-                               p.u_rank, rot, cmax, ec, eqw, thr);
+                               p.u_rank, rot, cmax, ec, eqw, thr, row_flag, fb.nflag);
         else if (n_groups <= 32 * kWave)
             hipLaunchKernelGGL(probe_threshold_wave_kernel<32>, wgrid, dim3(256), 0, s, gm, n_groups, nrows,
-                               p.u_rank, rot, cmax, ec, eqw, thr);
+                               p.u_rank, rot, cmax, ec, eqw, thr, row_flag, fb.nflag);
         else
             hipLaunchKernelGGL(probe_threshold_kernel, dim3(nrows), dim3(256), static_cast<size_t>(n_groups) * 4, s,
-                               gm, n_groups, nrows, p.u_rank, rot, cmax, ec, eqw, thr);
+                               gm, n_groups, nrows, p.u_rank, rot, cmax, ec, eqw, thr, row_flag, fb.nflag);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (part < 0 || part == 1) {
@@ -1342,10 +1356,10 @@ hipError_t launch_probe_mfma(hipStream_t s, const ProbePlan& p, const float* rot
         hipLaunchKernelGGL(probe_rerank_kernel, dim3((nrows + kRerankWaves - 1) / kRerankWaves),
                            dim3(kRerankWaves * kWave), static_cast<size_t>(kRerankWaves) * max_n * 8, s, rot, nrows,
                            centroids, norms, rv, rtile, cnt, p.lane_cap, 2 * p.splits, max_n, nprobe,
-                           p.u_rank >= nprobe, cmax, ec, eqw, row_flag, row_cand, labels);
+                           p.u_rank >= nprobe, cmax, ec, eqw, row_flag, row_cand, labels, fb.list, fb.nflag, fb.list_cap);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         // rows that overflowed or failed the check: exact recomputation
-        e = launch_probe_exact_flagged(s, rot, nrows, centroids, norms, k, nprobe, row_flag, labels, fb);
+        e = launch_probe_exact_flagged(s, rot, nrows, centroids, norms, k, nprobe, row_flag, labels, fb, true);
     }
     return e;
 }
@@ -1395,7 +1409,7 @@ hipError_t launch_assign_top1(hipStream_t s, const ProbePlan& p, const float* ro
     hipLaunchKernelGGL(probe_top1_rerank_kernel, dim3((nrows + kTop1Rows - 1) / kTop1Rows), dim3(256), 0, s, rows, nrows,
                        centroids, norms, buf, cnt, p.lane_cap, 2 * p.splits, cmax, ecmax, row_flag, labels);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    return launch_probe_exact_flagged(s, rows, nrows, centroids, norms, k, 1, row_flag, labels, fb);
+    return launch_probe_exact_flagged(s, rows, nrows, centroids, norms, k, 1, row_flag, labels, fb, false);
 }
 
 }  // namespace chimera

@@ -1,6 +1,7 @@
 // Query-side kernels: FhtKac rotation + QueryState + one-bit LUT, the exact
 // centroid probe, centroid norms and code unpacking.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -11,15 +12,18 @@ namespace chimera {
 // One wave per (query, token) row. Lane l holds elements l and l + 64.
 // Rotation: rotator.hpp:281-334. QueryState: chimera_index_internal.cuh:58-64
 // (sequential sum). LUT: kernels.cu:402-428, written as [q][c][e][i].
+// As the first kernel of a search it also clears the batch's status word.
 __global__ __launch_bounds__(256) void rotate_lut_kernel(const float* __restrict__ queries, int nq, int dim,
                                                          const uint8_t* __restrict__ flips, float fac, int ex_bits,
                                                          float* __restrict__ rot, float* __restrict__ cb1,
-                                                         float* __restrict__ cbex, float* __restrict__ lut) {
-    __shared__ float row[4][kDim];
+                                                         float* __restrict__ cbex, float* __restrict__ lut,
+                                                         uint32_t* __restrict__ status) {
+    __shared__ __align__(16) float row[4][kDim];
     __shared__ uint8_t fl[4 * kDim / 8];
     const int l = lane_id();
     const int w = wave_id();
     if (threadIdx.x < 4 * kDim / 8) fl[threadIdx.x] = flips[threadIdx.x];
+    if (status && blockIdx.x == 0 && threadIdx.x == 0) *status = 0u;
     __syncthreads();
     const int r = blockIdx.x * 4 + w;
     const bool valid = r < nq * kQ;
@@ -37,7 +41,14 @@ __global__ __launch_bounds__(256) void rotate_lut_kernel(const float* __restrict
     }
     if (l == 0) {
         float s = 0.0f;
-        for (int j = 0; j < kDim; ++j) s = s + row[w][j];
+#pragma unroll 8
+        for (int j = 0; j < kDim; j += 4) {
+            const float4 v = *reinterpret_cast<const float4*>(&row[w][j]);
+            s = s + v.x;
+            s = s + v.y;
+            s = s + v.z;
+            s = s + v.w;
+        }
         if (cb1) cb1[r] = s * ((1 << 1) - 1) / 2.0f;
         if (cbex) cbex[r] = s * ((1 << (ex_bits + 1)) - 1) / 2.0f;
     }
@@ -172,31 +183,16 @@ __device__ void exact_rows_topk(const float* q, const float* __restrict__ centro
 
 }  // namespace
 
-// Exact probe: for ROWS rotated query vectors per block, the nprobe
-// centroids with the smallest score (ties to the lower id), nearest first.
-// With row_flag, only blocks that hold a flagged row work; with gate, not
-// even those while *gate <= gate_cap (the split kernels below have taken
-// the flagged rows).
+namespace {
+
+// Exact labels of rows row0 .. row0 + ROWS - 1 over every centroid, by the
+// block; smem holds ROWS * cap keys and ROWS query rows.
 template <int ROWS>
-__global__ __launch_bounds__(256) void probe_exact_kernel(const float* __restrict__ rot, int nrows,
-                                                          const float* __restrict__ centroids,
-                                                          const float* __restrict__ norms, int64_t k, int nprobe,
-                                                          int cap, uint32_t* __restrict__ labels,
-                                                          const uint32_t* __restrict__ row_flag,
-                                                          const uint32_t* __restrict__ gate, int gate_cap) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    if (gate && *gate <= static_cast<uint32_t>(gate_cap)) return;
-    if (row_flag) {
-        bool any = false;
-        for (int rr = 0; rr < ROWS; ++rr)
-            if (blockIdx.x * ROWS + rr < nrows && row_flag[blockIdx.x * ROWS + rr]) any = true;
-        if (!any) return;
-    }
-    uint64_t* buf = reinterpret_cast<uint64_t*>(smem);                       // [ROWS][cap]
+__device__ void exact_row_block(const float* __restrict__ rot, int nrows, int row0, const float* __restrict__ centroids,
+                                const float* __restrict__ norms, int64_t k, int nprobe, int cap, unsigned char* smem,
+                                int* cnt, uint32_t* thr, uint32_t* __restrict__ labels) {
+    uint64_t* buf = reinterpret_cast<uint64_t*>(smem);                           // [ROWS][cap]
     float* q = reinterpret_cast<float*>(buf + static_cast<size_t>(ROWS) * cap);  // [ROWS][128]
-    __shared__ int cnt[ROWS];
-    __shared__ uint32_t thr[ROWS];  // ordered score threshold
-    const int row0 = blockIdx.x * ROWS;
     for (int t = threadIdx.x; t < ROWS * kDim; t += blockDim.x) {
         const int rr = t / kDim;
         q[t] = (row0 + rr < nrows) ? rot[static_cast<size_t>(row0 + rr) * kDim + (t % kDim)] : 0.0f;
@@ -209,6 +205,30 @@ __global__ __launch_bounds__(256) void probe_exact_kernel(const float* __restric
             labels[static_cast<size_t>(row0 + rr) * nprobe + p] =
                 static_cast<uint32_t>(buf[static_cast<size_t>(rr) * cap + p] & 0xFFFFFFFFu);
     }
+}
+
+}  // namespace
+
+// Exact probe: for ROWS rotated query vectors per block, the nprobe
+// centroids with the smallest score (ties to the lower id), nearest first.
+// With row_flag, only blocks that hold a flagged row work.
+template <int ROWS>
+__global__ __launch_bounds__(256) void probe_exact_kernel(const float* __restrict__ rot, int nrows,
+                                                          const float* __restrict__ centroids,
+                                                          const float* __restrict__ norms, int64_t k, int nprobe,
+                                                          int cap, uint32_t* __restrict__ labels,
+                                                          const uint32_t* __restrict__ row_flag) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ int cnt[ROWS];
+    __shared__ uint32_t thr[ROWS];  // ordered score threshold
+    const int row0 = static_cast<int>(blockIdx.x) * ROWS;
+    if (row_flag) {
+        bool any = false;
+        for (int rr = 0; rr < ROWS; ++rr)
+            if (row0 + rr < nrows && row_flag[row0 + rr]) any = true;
+        if (!any) return;
+    }
+    exact_row_block<ROWS>(rot, nrows, row0, centroids, norms, k, nprobe, cap, smem, cnt, thr, labels);
 }
 
 // The flagged rows in a list: list[f] for f < min(*nflag, list_cap), in no
@@ -261,18 +281,32 @@ __global__ __launch_bounds__(256) void probe_exact_split_kernel(const float* __r
     }
 }
 
-// Labels of listed row f from its splits' keys: all splits * nprobe keys
-// sorted in LDS (sort_n, a power of two, entries past them ~0), the first
-// nprobe ids written. One block per list entry.
-__global__ __launch_bounds__(256) void probe_exact_merge_kernel(const uint32_t* __restrict__ list,
-                                                                const uint32_t* __restrict__ nflag, int list_cap,
-                                                                const uint64_t* __restrict__ partial, int splits,
-                                                                int nprobe, int sort_n, uint32_t* __restrict__ labels) {
+// Labels of the flagged rows, after the split kernel. Block f takes listed
+// row f: all splits * nprobe keys sorted in LDS (sort_n, a power of two,
+// entries past them ~0), the first nprobe ids written. When more than
+// list_cap rows are flagged, block b takes rows b * ROWS .. b * ROWS +
+// ROWS - 1 over every centroid instead, if one of them is flagged.
+template <int ROWS>
+__global__ __launch_bounds__(256) void probe_exact_finish_kernel(
+    const float* __restrict__ rot, int nrows, const float* __restrict__ centroids, const float* __restrict__ norms,
+    int64_t k, int nprobe, int cap, const uint32_t* __restrict__ list, const uint32_t* __restrict__ nflag, int list_cap,
+    const uint64_t* __restrict__ partial, int splits, int sort_n, const uint32_t* __restrict__ row_flag,
+    uint32_t* __restrict__ labels) {
     extern __shared__ __align__(16) unsigned char smem[];
-    uint64_t* keys = reinterpret_cast<uint64_t*>(smem);  // [sort_n]
+    __shared__ int cnt[ROWS];
+    __shared__ uint32_t thr[ROWS];
     const uint32_t nf = *nflag;
+    if (nf > static_cast<uint32_t>(list_cap)) {
+        const int row0 = static_cast<int>(blockIdx.x) * ROWS;
+        bool any = false;
+        for (int rr = 0; rr < ROWS; ++rr)
+            if (row0 + rr < nrows && row_flag[row0 + rr]) any = true;
+        if (any) exact_row_block<ROWS>(rot, nrows, row0, centroids, norms, k, nprobe, cap, smem, cnt, thr, labels);
+        return;
+    }
+    uint64_t* keys = reinterpret_cast<uint64_t*>(smem);  // [sort_n]
     const uint32_t f = blockIdx.x;
-    if (nf > static_cast<uint32_t>(list_cap) || f >= nf) return;
+    if (f >= nf) return;
     const int n = splits * nprobe;
     for (int t = threadIdx.x; t < sort_n; t += blockDim.x)
         keys[t] = t < n ? partial[static_cast<size_t>(f) * n + t] : ~0ull;
@@ -343,27 +377,51 @@ __global__ void unpack_codes_kernel(int width, const uint8_t* __restrict__ packe
 
 // ---- host launchers ----
 
+namespace {
+
+// LDS of the exact kernels: ROWS * cap keys and ROWS query rows, and the
+// finish kernel's sort of splits * nprobe keys.
+size_t exact_lds(int rows, int cap) { return static_cast<size_t>(rows) * cap * 8 + static_cast<size_t>(rows) * kDim * 4; }
+
+int exact_sort_n(int nprobe) {
+    int n = 2;
+    while (n < exact_fallback_splits(nprobe) * nprobe) n <<= 1;
+    return n;
+}
+
+size_t finish_lds(int rows, int cap, int nprobe) {
+    return std::max(exact_lds(rows, cap), static_cast<size_t>(exact_sort_n(nprobe)) * 8);
+}
+
+int exact_rows(int cap) { return cap <= 1024 ? 8 : 2; }
+
+}  // namespace
+
 hipError_t configure_query_kernels(int nprobe) {
     const int cap = probe_buffer_cap(nprobe);
-    const int rows = cap <= 1024 ? 8 : 2;
-    const int shm = rows * cap * 8 + rows * kDim * 4;
-    if (shm <= 64 * 1024) return hipSuccess;
-    const void* whole = rows == 8 ? reinterpret_cast<const void*>(probe_exact_kernel<8>)
-                                  : reinterpret_cast<const void*>(probe_exact_kernel<2>);
-    const void* split = rows == 8 ? reinterpret_cast<const void*>(probe_exact_split_kernel<8>)
-                                  : reinterpret_cast<const void*>(probe_exact_split_kernel<2>);
-    const hipError_t e = hipFuncSetAttribute(whole, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+    const int rows = exact_rows(cap);
+    auto raise = [](const void* kernel, size_t bytes) {
+        if (bytes <= 64 * 1024) return hipSuccess;
+        return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+    };
+    const size_t shm = exact_lds(rows, cap);
+    hipError_t e = raise(rows == 8 ? reinterpret_cast<const void*>(probe_exact_kernel<8>)
+                                   : reinterpret_cast<const void*>(probe_exact_kernel<2>), shm);
     if (e != hipSuccess) return e;
-    return hipFuncSetAttribute(split, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+    e = raise(rows == 8 ? reinterpret_cast<const void*>(probe_exact_split_kernel<8>)
+                        : reinterpret_cast<const void*>(probe_exact_split_kernel<2>), shm);
+    if (e != hipSuccess) return e;
+    return raise(rows == 8 ? reinterpret_cast<const void*>(probe_exact_finish_kernel<8>)
+                           : reinterpret_cast<const void*>(probe_exact_finish_kernel<2>), finish_lds(rows, cap, nprobe));
 }
 
 hipError_t launch_rotate_lut(hipStream_t s, const float* queries, int nq, int dim, const uint8_t* flips,
-                             int ex_bits, float* rot, float* cb1, float* cbex, float* lut) {
+                             int ex_bits, float* rot, float* cb1, float* cbex, float* lut, uint32_t* status) {
     const int rows = nq * kQ;
     const int trunc = dim >= kDim ? kDim : 64;
     const float fac = 1.0F / sqrtf(static_cast<float>(trunc));
     hipLaunchKernelGGL(rotate_lut_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, queries, nq, dim, flips, fac,
-                       ex_bits, rot, cb1, cbex, lut);
+                       ex_bits, rot, cb1, cbex, lut, status);
     return hipGetLastError();
 }
 
@@ -381,25 +439,22 @@ int probe_buffer_cap(int nprobe) {
 
 static hipError_t launch_probe_exact_impl(hipStream_t s, const float* rot, int nrows, const float* centroids,
                                           const float* norms, int64_t k, int nprobe, uint32_t* labels,
-                                          const uint32_t* row_flag, const uint32_t* gate, int gate_cap) {
+                                          const uint32_t* row_flag) {
     const int cap = probe_buffer_cap(nprobe);
-    if (cap <= 1024) {
-        constexpr int R = 8;
-        const size_t shm = static_cast<size_t>(R) * cap * 8 + R * kDim * 4;
-        hipLaunchKernelGGL(probe_exact_kernel<R>, dim3((nrows + R - 1) / R), dim3(256), shm, s, rot, nrows,
-                           centroids, norms, k, nprobe, cap, labels, row_flag, gate, gate_cap);
-    } else {
-        constexpr int R = 2;
-        const size_t shm = static_cast<size_t>(R) * cap * 8 + R * kDim * 4;
-        hipLaunchKernelGGL(probe_exact_kernel<R>, dim3((nrows + R - 1) / R), dim3(256), shm, s, rot, nrows,
-                           centroids, norms, k, nprobe, cap, labels, row_flag, gate, gate_cap);
-    }
+    const int R = exact_rows(cap);
+    const dim3 grid((nrows + R - 1) / R);
+    if (R == 8)
+        hipLaunchKernelGGL(probe_exact_kernel<8>, grid, dim3(256), exact_lds(R, cap), s, rot, nrows, centroids, norms, k,
+                           nprobe, cap, labels, row_flag);
+    else
+        hipLaunchKernelGGL(probe_exact_kernel<2>, grid, dim3(256), exact_lds(R, cap), s, rot, nrows, centroids, norms, k,
+                           nprobe, cap, labels, row_flag);
     return hipGetLastError();
 }
 
 hipError_t launch_probe_exact(hipStream_t s, const float* rot, int nrows, const float* centroids,
                               const float* norms, int64_t k, int nprobe, uint32_t* labels) {
-    return launch_probe_exact_impl(s, rot, nrows, centroids, norms, k, nprobe, labels, nullptr, nullptr, 0);
+    return launch_probe_exact_impl(s, rot, nrows, centroids, norms, k, nprobe, labels, nullptr);
 }
 
 int exact_fallback_splits(int nprobe) {
@@ -408,44 +463,41 @@ int exact_fallback_splits(int nprobe) {
 
 hipError_t launch_probe_exact_flagged(hipStream_t s, const float* rot, int nrows, const float* centroids,
                                       const float* norms, int64_t k, int nprobe, const uint32_t* row_flag,
-                                      uint32_t* labels, const ExactFallback& fb) {
+                                      uint32_t* labels, const ExactFallback& fb, bool listed) {
     if (nrows <= 0) return hipSuccess;
     if (fb.list == nullptr || fb.list_cap <= 0 || nprobe > kExactPartialKeys)
-        return launch_probe_exact_impl(s, rot, nrows, centroids, norms, k, nprobe, labels, row_flag, nullptr, 0);
-    hipError_t e = launch_fill_u32(s, fb.nflag, 1, 0u);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(probe_flag_list_kernel, dim3((nrows + 255) / 256), dim3(256), 0, s, row_flag, nrows, fb.list,
-                       fb.nflag, fb.list_cap);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    // up to list_cap flagged rows: every centroid split of every ROWS of
-    // them in its own block, then one merge block per row (grids for at most
-    // nrows flagged rows: a one-query batch launches 32 merge blocks, not 512)
-    const int listed = std::min(fb.list_cap, nrows);
+        return launch_probe_exact_impl(s, rot, nrows, centroids, norms, k, nprobe, labels, row_flag);
+    hipError_t e = hipSuccess;
+    if (!listed) {
+        if ((e = launch_fill_u32(s, fb.nflag, 1, 0u)) != hipSuccess) return e;
+        hipLaunchKernelGGL(probe_flag_list_kernel, dim3((nrows + 255) / 256), dim3(256), 0, s, row_flag, nrows, fb.list,
+                           fb.nflag, fb.list_cap);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    // up to list_cap flagged rows: every centroid split of every R of them in
+    // its own block, then one merge block per row (grids for at most nrows
+    // flagged rows: a one-query batch launches 32 merge blocks, not 512);
+    // with more, the merge blocks take rows R at a time
+    const int rows = std::min(fb.list_cap, nrows);
     const int splits = exact_fallback_splits(nprobe);
     const int64_t chunk = (k + splits - 1) / splits;
     const int cap = probe_buffer_cap(nprobe);
-    if (cap <= 1024) {
-        constexpr int R = 8;
-        const size_t shm = static_cast<size_t>(R) * cap * 8 + R * kDim * 4;
-        hipLaunchKernelGGL(probe_exact_split_kernel<R>, dim3(splits, (listed + R - 1) / R), dim3(256), shm, s,
-                           rot, centroids, norms, k, nprobe, cap, fb.list, fb.nflag, fb.list_cap, chunk, splits,
-                           fb.partial);
-    } else {
-        constexpr int R = 2;
-        const size_t shm = static_cast<size_t>(R) * cap * 8 + R * kDim * 4;
-        hipLaunchKernelGGL(probe_exact_split_kernel<R>, dim3(splits, (listed + R - 1) / R), dim3(256), shm, s,
-                           rot, centroids, norms, k, nprobe, cap, fb.list, fb.nflag, fb.list_cap, chunk, splits,
-                           fb.partial);
-    }
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    int sort_n = 2;
-    while (sort_n < splits * nprobe) sort_n <<= 1;
-    hipLaunchKernelGGL(probe_exact_merge_kernel, dim3(listed), dim3(256), static_cast<size_t>(sort_n) * 8, s,
-                       fb.list, fb.nflag, fb.list_cap, fb.partial, splits, nprobe, sort_n, labels);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    // more flagged rows than the list holds: the row-block kernel
-    return launch_probe_exact_impl(s, rot, nrows, centroids, norms, k, nprobe, labels, row_flag, fb.nflag,
-                                   fb.list_cap);
+    const int R = exact_rows(cap);
+    const dim3 sgrid(splits, (rows + R - 1) / R);
+    const dim3 fgrid(std::max(rows, (nrows + R - 1) / R));
+    const int sort_n = exact_sort_n(nprobe);
+    auto run = [&](auto kk) {
+        constexpr int kR = decltype(kk)::value;
+        hipLaunchKernelGGL(probe_exact_split_kernel<kR>, sgrid, dim3(256), exact_lds(R, cap), s, rot, centroids, norms, k,
+                           nprobe, cap, fb.list, fb.nflag, fb.list_cap, chunk, splits, fb.partial);
+        const hipError_t se = hipGetLastError();
+        if (se != hipSuccess) return se;
+        hipLaunchKernelGGL(probe_exact_finish_kernel<kR>, fgrid, dim3(256), finish_lds(R, cap, nprobe), s, rot, nrows,
+                           centroids, norms, k, nprobe, cap, fb.list, fb.nflag, fb.list_cap, fb.partial, splits, sort_n,
+                           row_flag, labels);
+        return hipGetLastError();
+    };
+    return R == 8 ? run(std::integral_constant<int, 8>{}) : run(std::integral_constant<int, 2>{});
 }
 
 hipError_t launch_unpack_codes(hipStream_t s, int width, const uint8_t* packed, int64_t n, uint8_t* raw) {

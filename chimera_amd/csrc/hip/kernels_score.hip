@@ -893,14 +893,18 @@ __global__ __launch_bounds__(256) void fullbit_kernel(const float* __restrict__ 
 }
 
 // Final top-k (one 1,024-thread block per query): sort (SF, doc) descending.
+// With out_status the batch's status word goes along (no kernel after it).
 __global__ __launch_bounds__(1024) void final_topk_kernel(const int32_t* __restrict__ fcount,
                                                          const int32_t* __restrict__ fids,
                                                          const float* __restrict__ fscores, int fb_cap,
                                                          int sort_cap, int k, int64_t* __restrict__ out_ids,
                                                          float* __restrict__ out_scores,
-                                                         int32_t* __restrict__ out_counts) {
+                                                         int32_t* __restrict__ out_counts,
+                                                         const uint32_t* __restrict__ status,
+                                                         uint32_t* __restrict__ out_status) {
     extern __shared__ uint64_t keys[];
     const int q = blockIdx.x;
+    if (out_status && q == 0 && threadIdx.x == 0) *out_status = *status;
     const int cnt = fcount[q];
     const int n = cnt < 0 ? 0 : (cnt < fb_cap ? cnt : fb_cap);
     for (int t = threadIdx.x; t < sort_cap; t += blockDim.x) {
@@ -1024,11 +1028,11 @@ hipError_t launch_fullbit_mfma(hipStream_t s, int nq, const float* rot, const fl
 
 hipError_t launch_final_topk(hipStream_t s, int nq, const int32_t* fcount, const int32_t* fids,
                              const float* fscores, int fb_cap, int k, int64_t* out_ids, float* out_scores,
-                             int32_t* out_counts) {
+                             int32_t* out_counts, const uint32_t* status, uint32_t* out_status) {
     // at least one key per thread of the 1,024-thread block (its merge sort)
     const int sort_cap = std::max(pow2_at_least(fb_cap < 2 ? 2 : fb_cap), 1024);
     hipLaunchKernelGGL(final_topk_kernel, dim3(nq), dim3(1024), static_cast<size_t>(sort_cap) * 8, s, fcount, fids,
-                       fscores, fb_cap, sort_cap, k, out_ids, out_scores, out_counts);
+                       fscores, fb_cap, sort_cap, k, out_ids, out_scores, out_counts, status, out_status);
     return hipGetLastError();
 }
 
