@@ -86,6 +86,9 @@ struct Workspace {
     uint2* gsec = nullptr;        // [qs][nbk][groups_per_bucket(blog)]
     uint16_t* gkey = nullptr;     // [qs][nbk][groups_per_bucket(blog)]
     int32_t* ccount = nullptr;    // [qs] candidates per query
+    uint32_t* sel = nullptr;      // [split] split selection (see CandidateArgs)
+    uint64_t* sel_lists = nullptr;  // [split][select_list_cap(k_refine)]
+    int split = 0;
     int32_t* rcount = nullptr;    // [B]
     int32_t* rids = nullptr;      // [B * k_refine]
     float* rscore = nullptr;      // [B * k_refine]
@@ -101,6 +104,7 @@ struct Workspace {
 struct WorkspaceShape {
     size_t batch, qs, dim, nprobe, nbk, vcap, k_refine, fb_cap;
     bool staging;  // query staging and result counts of the host entry points
+    size_t split;  // queries of the split selection's state (0: none)
     int blog;      // documents per candidate bucket = 2^blog
 };
 
@@ -131,6 +135,11 @@ size_t carve_workspace(const WorkspaceShape& sh, unsigned char* base, Workspace*
     take(x.gsec, QS * sh.nbk * static_cast<size_t>(groups_per_bucket(sh.blog)));
     take(x.gkey, QS * sh.nbk * static_cast<size_t>(groups_per_bucket(sh.blog)));
     take(x.ccount, QS);
+    if (sh.split > 0) {
+        take(x.sel, sh.split * kSelectWords);
+        take(x.sel_lists, sh.split * static_cast<size_t>(select_list_cap(static_cast<int>(sh.k_refine))));
+    }
+    x.split = static_cast<int>(sh.split);
     take(x.rcount, B);
     take(x.rids, B * sh.k_refine);
     take(x.rscore, B * sh.k_refine);
@@ -539,6 +548,9 @@ CandidateArgs candidate_args(chimera_ctx* c, const Workspace& w) {
     a.err = w.err;
     a.num_cus = c->num_cus;
     a.wqs = w.qs;
+    a.sel = w.sel;
+    a.sel_lists = w.sel_lists;
+    a.sel_queries = w.split;
     return a;
 }
 
@@ -777,7 +789,8 @@ int finish_setup(chimera_ctx* c, const chimera_search_options& o, int32_t max_ba
 
     const WorkspaceShape sh{static_cast<size_t>(max_batch), static_cast<size_t>(c->qs), static_cast<size_t>(c->dim),
                             static_cast<size_t>(opt->nprobe), static_cast<size_t>(c->nbk), static_cast<size_t>(c->vcap),
-                            static_cast<size_t>(opt->k_refine), static_cast<size_t>(c->fb_cap), true, c->blog};
+                            static_cast<size_t>(opt->k_refine), static_cast<size_t>(c->fb_cap), true,
+                            static_cast<size_t>(std::min(c->qs, kSelectSplitQueries)), c->blog};
     unsigned char* block = nullptr;
     CK(dev_alloc(c, c->ws_allocs, &block, carve_workspace(sh, nullptr, nullptr), "search workspace"));
     carve_workspace(sh, block, &c->ws);
@@ -1165,7 +1178,7 @@ int chimera_search_device_noalloc(chimera_ctx* c, const float* d_queries, int32_
     const WorkspaceShape sh{static_cast<size_t>(nq), qs, static_cast<size_t>(c->dim),
                             static_cast<size_t>(c->opt.nprobe), static_cast<size_t>(c->nbk),
                             static_cast<size_t>(c->vcap), static_cast<size_t>(c->opt.k_refine),
-                            static_cast<size_t>(c->fb_cap), false, c->blog};
+                            static_cast<size_t>(c->fb_cap), false, 0, c->blog};
     const size_t need = carve_workspace(sh, nullptr, nullptr);
     if (need > kStaticScratchBytes) {
         // the largest batch that fits, for the message

@@ -131,7 +131,17 @@ struct CandidateArgs {
     uint32_t* err;
     int num_cus;
     int wqs;  // queries the candidate state (vcnt, vtot, rec, ...) holds
+    uint32_t* sel;        // [sel_queries][kSelectWords] split selection: S histogram, list count (null: not held)
+    uint64_t* sel_lists;  // [sel_queries][select_list_cap(k_refine)]
+    int sel_queries;
 };
+// Split selection: histogram bins, words of state per query (a multiple of
+// the 32 tokens), the most queries it holds state for, and the most documents
+// times queries of a sub-batch.
+constexpr int kSelectBins = 4096;
+constexpr int kSelectWords = kSelectBins + 32;
+constexpr int kSelectSplitQueries = 1024;
+constexpr int64_t kSelectSplitDocs = 8'000'000;
 int cand_buckets(int64_t num_docs, int blog);
 // Bucket size (log2) of the candidate stage for an index: the largest in
 // [kMinBucketLog2, kMaxBucketLog2] at which a (query, bucket) item expects at

@@ -202,13 +202,17 @@ __global__ __launch_bounds__(256) void cand_count_kernel(const uint32_t* __restr
                                                          int nprobe, const uint64_t* __restrict__ cluster_pos,
                                                          const int32_t* __restrict__ doc_clu, int64_t n_clusters,
                                                          int64_t num_docs, int blog, int nbk, int parts,
-                                                         uint32_t* __restrict__ vcnt) {
+                                                         uint32_t* __restrict__ vcnt, uint32_t* __restrict__ sel) {
     extern __shared__ uint32_t hist[];  // [nbk]
     __shared__ uint32_t runs[kMaxProbe];
     __shared__ uint32_t offs[kMaxProbe + 1];
     __shared__ int scratch[17];
     int qq, i, part;
     if (!cand_block(blockIdx.x, qs, parts, qq, i, part)) return;
+    if (sel && part == 0) {  // the 32 tokens' blocks clear the query's split selection
+        uint32_t* mine = sel + static_cast<size_t>(qq) * kSelectWords + static_cast<size_t>(i) * (kSelectWords / kQ);
+        for (int t = threadIdx.x; t < kSelectWords / kQ; t += blockDim.x) mine[t] = 0u;
+    }
     for (int t = threadIdx.x; t < nbk; t += blockDim.x) hist[t] = 0u;
     __syncthreads();
     const uint32_t* lab = labels + (static_cast<size_t>(q_base + qq) * kQ + i) * nprobe;
@@ -1032,6 +1036,138 @@ __global__ __launch_bounds__(kReduceThreads) void cand_reduce_dense_kernel(
 }
 
 
+// ---- split selection ----
+//
+// For small sub-batches the selection below (one block per query) would
+// leave most CUs idle while a block walks a query's candidates, a chain of
+// round trips: 61 us for one query over 300,000 documents and 95 us for 16
+// over 60,000, now 32 and 34 us. Its collection is spread over the GPU
+// instead: a histogram of every candidate's S (kSelectBins bins of
+// the float's top 16 bits from 2^-20 to 2^12; S is never negative), from
+// which each block of the next kernel takes the threshold T, the lower edge
+// of the bin of the R-th largest S, and lists the candidates at or above it.
+// The selection kernel then only sorts; it collects by itself when the list
+// overflows (ties, or scores outside the bins).
+namespace {
+
+constexpr uint32_t kSelectBase = (127u - 20u) << 7;  // top 16 bits of 2^-20
+
+__device__ __forceinline__ int select_bin(uint32_t bits) {
+    const int b = static_cast<int>(bits >> 16) - static_cast<int>(kSelectBase);
+    return b < 0 ? 0 : (b < kSelectBins ? b : kSelectBins - 1);
+}
+
+// f(candidate) over the candidates of the block's share of the query's
+// buckets: a wave takes a 2^-sub_log part of a bucket at a time, four loads
+// in flight. The candidates of a bucket are contiguous.
+template <typename F>
+__device__ __forceinline__ void for_each_candidate(const uint32_t* __restrict__ tq, const uint32_t* __restrict__ offq,
+                                                   const uint2* __restrict__ rq, int nbk, int bshift, int sub_log,
+                                                   F&& f) {
+    const int lane = lane_id();
+    const int nwaves = static_cast<int>(gridDim.x * blockDim.x) / kWave;
+    const int w0 = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+    for (int unit = w0; unit < (nbk << sub_log); unit += nwaves) {
+        const int b = unit >> sub_log;
+        const int64_t n = tq[b];
+        const int part = unit & ((1 << sub_log) - 1);
+        const int first = static_cast<int>((n * part) >> sub_log), end = static_cast<int>((n * (part + 1)) >> sub_log);
+        const uint2* src = rq + offq[static_cast<size_t>(b) << bshift];
+        for (int j0 = first; j0 < end; j0 += 4 * kWave) {
+            uint2 e[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int j = j0 + u * kWave + lane;
+                e[u] = src[j < end ? j : first];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (j0 + u * kWave + lane < end) f(e[u]);
+        }
+    }
+}
+
+}  // namespace
+
+__global__ __launch_bounds__(256) void select_hist_kernel(const uint32_t* __restrict__ vcnt,
+                                                          const uint32_t* __restrict__ tcount,
+                                                          const uint2* __restrict__ rec, int64_t vcap, int nbk,
+                                                          int bshift, int sub_log, uint32_t* __restrict__ sel) {
+    __shared__ uint32_t hist[kSelectBins];
+    const int qq = blockIdx.y;
+    for (int t = threadIdx.x; t < kSelectBins; t += blockDim.x) hist[t] = 0u;
+    __syncthreads();
+    for_each_candidate(tcount + static_cast<size_t>(qq) * nbk, vcnt + (static_cast<size_t>(qq) * nbk << bshift),
+                       rec + static_cast<size_t>(qq) * vcap, nbk, bshift, sub_log,
+                       [&](const uint2& e) { atomicAdd(&hist[select_bin(e.y)], 1u); });
+    __syncthreads();
+    uint32_t* out = sel + static_cast<size_t>(qq) * kSelectWords;
+    for (int t = threadIdx.x; t < kSelectBins; t += blockDim.x)
+        if (hist[t] != 0u) atomicAdd(&out[t], hist[t]);
+}
+
+// Lists the candidates with S >= T (at most list_cap; the count, which may
+// exceed it, in word kSelectBins of sel), in no particular order.
+__global__ __launch_bounds__(256) void select_collect_kernel(const uint32_t* __restrict__ vcnt,
+                                                             const uint32_t* __restrict__ tcount,
+                                                             const uint2* __restrict__ rec, int64_t vcap, int nbk,
+                                                             int bshift, int sub_log, int k_refine, int list_cap,
+                                                             uint32_t* __restrict__ sel, uint64_t* __restrict__ lists) {
+    __shared__ int scratch[17];
+    __shared__ int s_bin;
+    __shared__ int s_base;
+    const int qq = blockIdx.y;
+    uint32_t* hist = sel + static_cast<size_t>(qq) * kSelectWords;
+    // bins from the top: thread t holds bins top - 15 .. top of its run
+    constexpr int kPer = kSelectBins / 256;
+    const int top = kSelectBins - 1 - kPer * static_cast<int>(threadIdx.x);
+    int own[kPer];
+    int mine = 0;
+#pragma unroll
+    for (int u = 0; u < kPer; u += 4) {
+        const uint4 v = *reinterpret_cast<const uint4*>(&hist[top - u - 3]);
+        own[u] = static_cast<int>(v.w);
+        own[u + 1] = static_cast<int>(v.z);
+        own[u + 2] = static_cast<int>(v.y);
+        own[u + 3] = static_cast<int>(v.x);
+        mine += own[u] + own[u + 1] + own[u + 2] + own[u + 3];
+    }
+    if (threadIdx.x == 0) s_bin = 0;
+    int C;
+    const int incl = block_inclusive_scan_shared(mine, scratch, &C);
+    const int R = C < k_refine ? C : k_refine;
+    if (C > list_cap && incl >= R && incl - mine < R) {  // this thread's run holds the R-th largest
+        int cum = incl - mine;
+        for (int u = 0; u < kPer; ++u) {
+            cum += own[u];
+            if (cum >= R) {
+                s_bin = top - u;
+                break;
+            }
+        }
+    }
+    __syncthreads();
+    const int bin = s_bin;
+    const uint32_t T = bin == 0 ? 0u : (kSelectBase + static_cast<uint32_t>(bin)) << 16;
+    const uint32_t* tq = tcount + static_cast<size_t>(qq) * nbk;
+    const uint32_t* offq = vcnt + (static_cast<size_t>(qq) * nbk << bshift);
+    const uint2* rq = rec + static_cast<size_t>(qq) * vcap;
+    // counted first, so that one atomic per block takes the block's places
+    int n = 0;
+    for_each_candidate(tq, offq, rq, nbk, bshift, sub_log, [&](const uint2& e) { n += e.y >= T ? 1 : 0; });
+    int total;
+    const int before = block_inclusive_scan_shared(n, scratch, &total) - n;
+    if (threadIdx.x == 0) s_base = total > 0 ? static_cast<int>(atomicAdd(&hist[kSelectBins], static_cast<uint32_t>(total))) : 0;
+    __syncthreads();
+    int slot = s_base + before;
+    uint64_t* list = lists + static_cast<size_t>(qq) * list_cap;
+    for_each_candidate(tq, offq, rq, nbk, bshift, sub_log, [&](const uint2& e) {
+        if (e.y < T) return;
+        if (slot < list_cap) list[slot] = (static_cast<uint64_t>(~float_to_ordered(__uint_as_float(e.y))) << 32) | e.x;
+        ++slot;
+    });
+}
+
 // Top R = min(k_refine, C) candidates of one query by (S desc, doc asc).
 // Any T at or below the R-th largest group maximum bounds the R-th largest
 // S from below (each group maximum is the S of a distinct candidate), so the
@@ -1051,13 +1187,14 @@ __global__ __launch_bounds__(kReduceThreads) void cand_reduce_dense_kernel(
 // fills and at the end of the walk. Two 1,024-thread blocks share a CU (LDS), which
 // holds only while the kernel uses at most 80 SGPRs per wave, a limit the
 // compiler's occupancy model does not apply; amdgpu_num_sgpr keeps it.
+// With `sel`, the split selection has listed the candidates in `lists`.
 template <int kBlog>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80))) void select_refine_kernel(
     const uint32_t* __restrict__ vcnt, const uint32_t* __restrict__ tcount, const float2* __restrict__ gstat,
     const uint2* __restrict__ gsec, const uint16_t* __restrict__ gkey, const uint2* __restrict__ rec, int64_t vcap,
     int nbk, int bshift, int q_base, int qs, int k_refine, int list_cap,
     int32_t* __restrict__ ccount, int32_t* __restrict__ rcount, int32_t* __restrict__ rids,
-    float* __restrict__ rscore) {
+    float* __restrict__ rscore, const uint32_t* __restrict__ sel, const uint64_t* __restrict__ lists) {
     constexpr int kGpb = groups_per_bucket(kBlog);
     extern __shared__ uint64_t list[];  // [list_cap]
     __shared__ __align__(16) int hist[256];
@@ -1090,8 +1227,13 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80))) void sel
     }
     if (R == 0) return;
     const bool take_all = C <= list_cap;
+    const int listed = sel ? static_cast<int>(sel[static_cast<size_t>(qq) * kSelectWords + kSelectBins]) : list_cap + 1;
     uint32_t T = 0u;
-    if (!take_all) {
+    if (listed <= list_cap) {
+        const uint64_t* pre = lists + static_cast<size_t>(qq) * list_cap;
+        for (int t = threadIdx.x; t < listed; t += blockDim.x) list[t] = pre[t];
+        if (threadIdx.x == 0) s_n = listed;
+    } else if (!take_all) {
         const int64_t G = static_cast<int64_t>(nbk) * kGpb;
         const uint16_t* kq = gkey + static_cast<size_t>(qq) * nbk * kGpb;
         T = block_radix_select<true, 2>([&](int64_t g) { return static_cast<uint32_t>(kq[g]) << 16; }, G, R, hist,
@@ -1449,11 +1591,24 @@ static int log2_of(int p) {
     return l;
 }
 
+// Whether a sub-batch of qs queries takes the split selection: its candidates
+// (at most a document each, read three times) are few enough, and either the
+// groups cannot prune (fewer than 4 k_refine of them, so the query-per-block
+// kernel walks every candidate) or it leaves half of the CUs idle. A search
+// of 52 queries over 150,000 documents (7.8M documents times queries, groups
+// that do not prune): 1,736 us without, 1,466 with; 26 over 300,000: 1,010
+// and 975; 300 over 150,000 (45M): 7,331 and 7,531.
+static bool select_split(const CandidateArgs& a, int qs) {
+    if (a.sel == nullptr || qs > a.sel_queries || static_cast<int64_t>(qs) * a.num_docs > kSelectSplitDocs) return false;
+    const int64_t groups = static_cast<int64_t>(a.nbk) * groups_per_bucket(a.blog);
+    return groups < 4 * static_cast<int64_t>(a.k_refine) || qs <= a.num_cus / 2;
+}
+
 template <int kBlog>
 static void launch_select(hipStream_t s, const CandidateArgs& a, int bshift, int q_base, int qs, int cap) {
     hipLaunchKernelGGL(select_refine_kernel<kBlog>, dim3(qs), dim3(1024), static_cast<size_t>(cap) * 8, s, a.vcnt,
                        a.tcount, a.gstat, a.gsec, a.gkey, a.rec, a.vcap, a.nbk, bshift, q_base, qs, a.k_refine, cap,
-                       a.ccount, a.rcount, a.rids, a.rscore);
+                       a.ccount, a.rcount, a.rids, a.rscore, select_split(a, qs) ? a.sel : nullptr, a.sel_lists);
 }
 
 hipError_t launch_candidates(hipStream_t s, const CandidateArgs& a, int q_base, int qs, int phase) {
@@ -1466,7 +1621,8 @@ hipError_t launch_candidates(hipStream_t s, const CandidateArgs& a, int q_base, 
     switch (phase) {
         case 0:
             hipLaunchKernelGGL(cand_count_kernel, dim3(grid), dim3(256), shm, s, a.labels, q_base, qs, a.nprobe,
-                               a.cluster_pos, a.doc_clu, a.n_clusters, a.num_docs, a.blog, a.nbk, parts, a.vcnt);
+                               a.cluster_pos, a.doc_clu, a.n_clusters, a.num_docs, a.blog, a.nbk, parts, a.vcnt,
+                               select_split(a, qs) ? a.sel : nullptr);
             break;
         case 1: {
             const int nseg = offsets_segments(qs, a.num_cus, a.nbk * kQ * parts / 4, a.vcap);
@@ -1519,6 +1675,17 @@ hipError_t launch_candidates(hipStream_t s, const CandidateArgs& a, int q_base, 
             break;
         case 4: {
             const int cap = select_list_cap(a.k_refine);
+            if (select_split(a, qs)) {
+                // parts of at most 512 documents, a wave each, over about two
+                // blocks per CU (at least one per query)
+                const int sub_log = std::max(0, a.blog - 9);
+                const int64_t units = static_cast<int64_t>(a.nbk) << sub_log;
+                const int nb = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>((units + 3) / 4, std::max(1, 2 * a.num_cus / qs))));
+                hipLaunchKernelGGL(select_hist_kernel, dim3(nb, qs), dim3(256), 0, s, a.vcnt, a.tcount, a.rec, a.vcap,
+                                   a.nbk, bshift, sub_log, a.sel);
+                hipLaunchKernelGGL(select_collect_kernel, dim3(nb, qs), dim3(256), 0, s, a.vcnt, a.tcount, a.rec, a.vcap,
+                                   a.nbk, bshift, sub_log, a.k_refine, cap, a.sel, a.sel_lists);
+            }
             switch (a.blog) {
                 case 8: launch_select<8>(s, a, bshift, q_base, qs, cap); break;
                 case 9: launch_select<9>(s, a, bshift, q_base, qs, cap); break;
