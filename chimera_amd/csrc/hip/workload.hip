@@ -2,6 +2,8 @@
 // (include/chimera_workload.h).
 #include "capi_internal.hpp"
 #include "chimera_workload.h"
+#include <algorithm>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -227,12 +229,14 @@ __device__ __forceinline__ void load_query_split(const float* __restrict__ query
 // tile's rows is scaled back by 2^-st, the document's max by 2^-sq.
 // One tile's loads at a time: three waves per SIMD hide their latency
 // (a second tile in registers would leave two).
-// Rows past the end read the last token and are masked; -inf for an empty
-// document; every lane gets the value.
-__device__ __forceinline__ float doc_maxsim_split(const float* __restrict__ emb, int start, int end,
-                                                  const half8_t (&bq)[4][2][2], const float (&inv)[2], int c,
-                                                  int g) {
-    float mx0 = -INFINITY, mx1 = -INFINITY;
+// Rows past the end read the last token and are masked. The tiles of
+// [start, end) from first on, `step` tokens apart: their maxima per lane in
+// mx0 and mx1 (-inf without a tile); maxsim_finish makes them the document's
+// score.
+__device__ __forceinline__ void doc_maxsim_tiles(const float* __restrict__ emb, int start, int end, int first, int step,
+                                                 const half8_t (&bq)[4][2][2], int c, int g, float& mx0, float& mx1) {
+    mx0 = -INFINITY;
+    mx1 = -INFINITY;
     auto load = [&](int t0, float (&a)[32]) {
         const int tok = t0 + c < end ? t0 + c : end - 1;
         const float4* src = reinterpret_cast<const float4*>(emb + static_cast<size_t>(tok) * kDim + 32 * g);
@@ -284,11 +288,16 @@ __device__ __forceinline__ float doc_maxsim_split(const float* __restrict__ emb,
         mx0 = fmaxf(mx0, t0m * is);
         mx1 = fmaxf(mx1, t1m * is);
     };
-    for (int t0 = start; t0 < end; t0 += 16) {
+    for (int t0 = start + first; t0 < end; t0 += step) {
         float a0[32];
         load(t0, a0);
         tile(a0, t0);
     }
+}
+
+// Score of a document from its tiles' maxima, in every lane; -inf for an
+// empty document.
+__device__ __forceinline__ float maxsim_finish(float mx0, float mx1, const float (&inv)[2]) {
     mx0 = fmaxf(mx0, __shfl_xor(mx0, 16, kWave));
     mx0 = fmaxf(mx0, __shfl_xor(mx0, 32, kWave));
     mx1 = fmaxf(mx1, __shfl_xor(mx1, 16, kWave));
@@ -329,11 +338,68 @@ __global__ __launch_bounds__(kRescoreWaves * kWave) void maxsim_rescore_kernel(
     for (int j = j0 + wave_id(); j < j1; j += kRescoreWaves) {
         const int32_t d = cand_ids[static_cast<size_t>(q) * cap + j];
         float v = -INFINITY;
-        if (d >= 0 && d < m) v = doc_maxsim_split(emb, doc_ptrs[d], doc_ptrs[d + 1], bq, inv, c, g);
+        if (d >= 0 && d < m) {
+            float mx0, mx1;
+            doc_maxsim_tiles(emb, doc_ptrs[d], doc_ptrs[d + 1], 0, 16, bq, c, g, mx0, mx1);
+            v = maxsim_finish(mx0, mx1, inv);
+        }
         if (l == 0) scores[static_cast<size_t>(q) * cap + j] = v;
     }
 }
 
+// The same scores for few candidates: `split` waves of the block share a
+// document (tile t of it goes to wave t mod split), so that its tiles are
+// loaded side by side; their maxima meet in LDS. What bounds a small call is
+// the round trip per tile of the longest document: one query of 100
+// candidates of up to 256 tokens took 57 us with a wave per document, 11 with eight.
+constexpr int kRescoreSmallWaves = 8;
+__global__ __launch_bounds__(kRescoreSmallWaves * kWave) void maxsim_rescore_small_kernel(
+    const float* __restrict__ emb, const int32_t* __restrict__ doc_ptrs, int64_t m, const float* __restrict__ queries,
+    const int32_t* __restrict__ cand_ids, const int32_t* __restrict__ cand_counts, int cap, int split,
+    float* __restrict__ scores) {
+    __shared__ float part[kRescoreSmallWaves][2][kWave];
+    const int q = blockIdx.y;
+    const int cnt = cand_counts[q];
+    const int n = cnt < 0 ? 0 : (cnt < cap ? cnt : cap);
+    const int per = static_cast<int>(blockDim.x) / kWave / split;
+    if (static_cast<int>(blockIdx.x) * per >= n) return;
+    const int l = lane_id();
+    const int w = wave_id();
+    const int c = l & 15;
+    const int g = l >> 4;
+    const int j = static_cast<int>(blockIdx.x) * per + w / split;
+    const int32_t d = j < n ? cand_ids[static_cast<size_t>(q) * cap + j] : -1;
+    // waves past the document's tiles only meet at the barrier
+    const bool in = d >= 0 && d < m;
+    const int start = in ? doc_ptrs[d] : 0, end = in ? doc_ptrs[d + 1] : 0;
+    const int mine = w % split;
+    float inv[2] = {0.0f, 0.0f};
+    float mx0 = -INFINITY, mx1 = -INFINITY;
+    if (start + 16 * mine < end) {
+        half8_t bq[4][2][2];
+        load_query_split(queries + static_cast<size_t>(q) * kQ * kDim, c, g, bq, inv);
+        doc_maxsim_tiles(emb, start, end, 16 * mine, 16 * split, bq, c, g, mx0, mx1);
+    }
+    part[w][0][l] = mx0;
+    part[w][1][l] = mx1;
+    __syncthreads();
+    if (mine != 0 || j >= n) return;
+    for (int o = 1; o < split; ++o) {
+        mx0 = fmaxf(mx0, part[w + o][0][l]);
+        mx1 = fmaxf(mx1, part[w + o][1][l]);
+    }
+    const float v = start < end ? maxsim_finish(mx0, mx1, inv) : -INFINITY;
+    if (l == 0) scores[static_cast<size_t>(q) * cap + j] = v;
+}
+
+// Calls of up to this many candidate documents share each document between
+// waves: eight while that is at most 16 waves a CU, else four. Whole calls
+// with documents of up to 256 tokens: 100 candidates 72 -> 28 us, 900 95 ->
+// 43, 1,800 95 -> 57; of up to 32 tokens: 33 -> 24, 33 -> 30, 34.5 -> 34.6.
+// Past 2,048 the short ones lose (3,000: 36 -> 39 us), as every block loads
+// its query.
+constexpr int64_t kRescoreSmallDocs = 2048;
+int rescore_split(int64_t docs) { return docs <= 512 ? 8 : 4; }
 
 // Matrix-core throughput with register operands: every wave runs `iters`
 // rounds of independent accumulation chains of one instruction type on
@@ -504,11 +570,20 @@ int chimera_maxsim_rescore_device(chimera_ctx* ctx, const float* d_embeddings, c
     if (!d_embeddings || !d_doc_ptrs || !d_queries || !d_cand_ids || !d_cand_counts || !d_cand_scores)
         return api_fail(CHIMERA_ERR_INVALID_ARGUMENT, "null argument");
     if (k > 0 && (!d_top_ids || !d_top_counts)) return api_fail(CHIMERA_ERR_INVALID_ARGUMENT, "null top-k output");
-    const dim3 grid(static_cast<unsigned>((cand_cap + kRescoreDocsPerBlock - 1) / kRescoreDocsPerBlock),
-                    static_cast<unsigned>(nq));
     stage_begin(ctx, kStageRescore);
-    hipLaunchKernelGGL(maxsim_rescore_kernel, grid, dim3(kRescoreWaves * kWave), 0, s, d_embeddings, d_doc_ptrs,
-                       num_docs, d_queries, d_cand_ids, d_cand_counts, cand_cap, d_cand_scores);
+    const int64_t docs = static_cast<int64_t>(nq) * cand_cap;
+    if (docs <= kRescoreSmallDocs) {
+        const int split = rescore_split(docs);
+        const int waves = std::max(split, 4);
+        const int per = waves / split;
+        hipLaunchKernelGGL(maxsim_rescore_small_kernel, dim3((cand_cap + per - 1) / per, nq), dim3(waves * kWave), 0, s, d_embeddings, d_doc_ptrs, num_docs, d_queries,
+                           d_cand_ids, d_cand_counts, cand_cap, split, d_cand_scores);
+    } else {
+        const dim3 grid(static_cast<unsigned>((cand_cap + kRescoreDocsPerBlock - 1) / kRescoreDocsPerBlock),
+                        static_cast<unsigned>(nq));
+        hipLaunchKernelGGL(maxsim_rescore_kernel, grid, dim3(kRescoreWaves * kWave), 0, s, d_embeddings, d_doc_ptrs,
+                           num_docs, d_queries, d_cand_ids, d_cand_counts, cand_cap, d_cand_scores);
+    }
     hipError_t e = hipGetLastError();
     stage_end(ctx);
     if (e != hipSuccess) return api_fail(CHIMERA_ERR_HIP, std::string("MaxSim rescoring kernel failed: ") + hipGetErrorString(e));
