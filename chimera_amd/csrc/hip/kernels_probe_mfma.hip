@@ -205,7 +205,15 @@ __global__ __launch_bounds__(256) void probe_centroids_kernel(const float* __res
 // Slots of tiles past the split or past k load centroid 0 and get the
 // initial value -inf, which makes every accumulator of theirs -inf: never
 // a hit and never a minimum.
-template <int MODE, int G = kGroupTiles>
+//
+// TS (MODE 0 and 1): waves that share 64 rows. With few rows (at most 512 /
+// TS) the block's other waves would only help staging, so TS of them take the
+// tiles of a stage in turn: tile t goes to wave t mod TS of the row group.
+// Their hits append to the same sub-lists through counters in LDS (the
+// rerank sorts, so the order of records is free), and the tile minima of a
+// stage meet in LDS. One query over 262,144 centroids: filtered pass 34 -> 22
+// us (3.0 TB/s of centroids), sampled pass 11.7 -> 10.6.
+template <int MODE, int G = kGroupTiles, int TS = 1>
 __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
     const float* __restrict__ rot, int nrows, const uint16_t* __restrict__ cbf, const float* __restrict__ nhalf,
     int64_t k, int tiles_per_split, int sample_stride, float* __restrict__ gm, const float* __restrict__ thr,
@@ -216,11 +224,21 @@ __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
     __shared__ __align__(16) unsigned char stage1[kStageTiles * kTileBytes];
     __shared__ __align__(16) float snorm0[kStageTiles * 32];
     __shared__ __align__(16) float snorm1[kStageTiles * 32];
-    __shared__ float gbuf[MODE == 0 ? kRowsPerBlock * 8 : 1];  // MODE 0: [row of the block][column mod 8]
+    // MODE 0: [row of the block][column mod 8] (TS > 1: [row][tile of the stage])
+    __shared__ float gbuf[MODE == 0 ? kRowsPerBlock / TS * 8 : 1];
+    // MODE 1, TS > 1: records of each (row of the block, lane half)
+    __shared__ int scnt[MODE == 1 && TS > 1 ? kRowsPerBlock / TS * 2 : 1];
+    static_assert(TS == 1 || MODE <= 1, "only the probe's passes share rows between waves");
+    static_assert(kStageTiles % TS == 0 && kProbeWaves % TS == 0, "whole turns");
     const int l = lane_id();
     const int w = wave_id();
+    const int wr = w / TS;      // row group of the wave
+    const int phase = w % TS;   // its first tile of a stage
     const int j = l & 31;
     const int hk = l >> 5;  // k half within a 16-wide k step
+    if (MODE == 1 && TS > 1) {
+        for (int t = threadIdx.x; t < kRowsPerBlock / TS * 2; t += blockDim.x) scnt[t] = 0;  // seen after the first barrier
+    }
     // 1-D grid of row_blocks * splits blocks. The XCDs take block ids
     // round-robin; with splits a multiple of 8, XCD x runs only splits x,
     // x + 8, ..., row blocks fastest, so the blocks resident on one XCD stream
@@ -234,7 +252,7 @@ __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
         rb = static_cast<int>(blockIdx.x) % row_blocks;
         sp = static_cast<int>(blockIdx.x) / row_blocks;
     }
-    const int row0 = rb * kRowsPerBlock + w * kRowsPerWave;
+    const int row0 = rb * (kRowsPerBlock / TS) + wr * kRowsPerWave;
     const int64_t ntiles = (k + 31) / 32;
     const int64_t n_sampled = (ntiles + sample_stride - 1) / sample_stride;
     static_assert(kStageTiles % G == 0, "whole groups per stage");
@@ -356,6 +374,8 @@ __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
                 m = wave_max_xor32(m);
                 if (MODE == 2) {
                     rmax[cb] = fmaxf(rmax[cb], m);
+                } else if (TS > 1) {
+                    if (hk == 0) gbuf[(wr * kRowsPerWave + 32 * cb + j) * 8 + tt] = m;
                 } else {
                     gmax[cb][tt / G] = fmaxf(gmax[cb][tt / G], m);
                 }
@@ -363,6 +383,7 @@ __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
                 // a lane with a hit stores its whole tile column (no
                 // per-value tests here: the rerank does them)
                 const bool hit = m >= th[cb];  // th is +inf past the last row
+                if (TS > 1 && hit) lcnt[cb] = atomicAdd(&scnt[(wr * kRowsPerWave + 32 * cb + j) * 2 + hk], 1);
                 if (hit && lcnt[cb] < lane_cap) {
                     const size_t e = sub[cb] + static_cast<size_t>(lcnt[cb]);
                     const float t = th[cb];
@@ -372,7 +393,7 @@ __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
                     dv[1] = make_uint4(pk(8), pk(10), pk(12), pk(14));
                     rtile[e] = static_cast<uint32_t>(tile);
                 }
-                lcnt[cb] += hit ? 1 : 0;
+                if (TS == 1) lcnt[cb] += hit ? 1 : 0;
             } else if (m >= th[cb]) {  // MODE 3; th is +inf past the last row
                 // the lane's best so far bounds the nearest d' too
                 th[cb] = fmaxf(th[cb], m - dl[cb]);
@@ -417,14 +438,16 @@ __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
         // tile replaces fragment s of this one once the second chain has
         // issued its MFMA s, eight MFMAs before the next tile needs it.
         float16_t acc1;
-        float16_t nx = ninit(0);
+        float16_t nx = ninit(phase);
         bf16x8_t a[8];
 #pragma unroll
-        for (int s = 0; s < 8; ++s) a[s] = load_a(0, s);
+        for (int s = 0; s < 8; ++s) a[s] = load_a(phase, s);
+        constexpr int kTurns = kStageTiles / TS;
 #pragma unroll
-        for (int tt = 0; tt < kStageTiles; ++tt) {
+        for (int i = 0; i < kTurns; ++i) {
+            const int tt = phase + i * TS;
             const int64_t tile = tile_of(iter * kStageTiles + tt);
-            const bool more = tt + 1 < kStageTiles;
+            const bool more = i + 1 < kTurns;
             // Skewed schedule: the check of one column block's tile runs
             // after the other column block's MFMA chain has been issued, so
             // its results are ready and the matrix cores are not left idle
@@ -434,21 +457,21 @@ __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
             float16_t acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], bq[0][0], nx, 0, 0, 0);
 #pragma unroll
             for (int s = 1; s < 8; ++s) acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s], bq[0][s], acc0, 0, 0, 0);
-            if (tt > 0) check(1, acc1, tile - sample_stride, tt - 1);
+            if (i > 0) check(1, acc1, tile - TS * sample_stride, tt - TS);
             acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], bq[1][0], nx, 0, 0, 0);
             if (more) {
-                nx = ninit(tt + 1);
-                a[0] = load_a(tt + 1, 0);
+                nx = ninit(tt + TS);
+                a[0] = load_a(tt + TS, 0);
             }
 #pragma unroll
             for (int s = 1; s < 8; ++s) {
                 acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s], bq[1][s], acc1, 0, 0, 0);
-                if (more) a[s] = load_a(tt + 1, s);
+                if (more) a[s] = load_a(tt + TS, s);
             }
             check(0, acc0, tile, tt);
         }
-        check(1, acc1, tile_of(iter * kStageTiles + kStageTiles - 1), kStageTiles - 1);
-        if (MODE == 0) {
+        check(1, acc1, tile_of(iter * kStageTiles + phase + (kTurns - 1) * TS), phase + (kTurns - 1) * TS);
+        if (MODE == 0 && TS == 1) {
             // The wave's group minima gather in LDS and leave as runs of up
             // to 8 consecutive groups per row (32-byte writes instead of
             // scattered 4-byte ones); runs end at multiples of 8 columns.
@@ -482,17 +505,41 @@ __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
     // wave's own loads have landed (vmcnt 0) and the barrier makes every
     // wave's visible; it also ends the reads of the other buffer, which the
     // loads of the next stage then overwrite.
+    // MODE 0, TS > 1: the stage's group minima, once every wave's tiles are in
+    // (the barrier at the top of the next stage ends these reads)
+    auto flush = [&](int64_t iter) {
+        if (MODE != 0 || TS == 1) return;
+        __syncthreads();
+        const int64_t col = gcol0 + kGroupsPerStage * iter;
+        const int rows = nrows - rb * (kRowsPerBlock / TS);
+        for (int v = threadIdx.x; v < kRowsPerBlock / TS * kGroupsPerStage; v += blockDim.x) {
+            const int rl = v / kGroupsPerStage, h = v % kGroupsPerStage;
+            if (rl >= rows || col + h >= n_groups) continue;
+            float m = gbuf[rl * 8 + h * G];
+#pragma unroll
+            for (int u = 1; u < G; ++u) m = fmaxf(m, gbuf[rl * 8 + h * G + u]);
+            gm[static_cast<size_t>(rb * (kRowsPerBlock / TS) + rl) * n_groups + col + h] = -2.0f * m;
+        }
+    };
     if (n_iter > 0) fetch(0, stage0, snorm0);
     for (int64_t iter = 0; iter < n_iter; iter += 2) {
         __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
         __syncthreads();
         if (iter + 1 < n_iter) fetch(iter + 1, stage1, snorm1);
         compute(iter, stage0, snorm0);
+        flush(iter);
         if (iter + 1 >= n_iter) break;
         __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
         __syncthreads();
         if (iter + 2 < n_iter) fetch(iter + 2, stage0, snorm0);
         compute(iter + 1, stage1, snorm1);
+        flush(iter + 1);
+    }
+    if (MODE == 1 && TS > 1) {
+        __syncthreads();
+        if (phase != 0) return;
+#pragma unroll
+        for (int cb = 0; cb < kColBlocks; ++cb) lcnt[cb] = scnt[(wr * kRowsPerWave + 32 * cb + j) * 2 + hk];
     }
     if (MODE == 2) {
 #pragma unroll
@@ -756,10 +803,11 @@ __global__ __launch_bounds__(256) void probe_threshold_kernel(const float* __res
 }
 
 // The same U and thr with one wave per row and the row's minima in registers
-// (kPerLane per lane, for rows of at most 64 kPerLane minima): four 8-bit
-// radix passes over the ordered keys, each a wave-local histogram (lanes that
-// share the first active lane's digit add through it) and a scan of its bins
-// (lane L holds bins 4L .. 4L + 3), with no block barriers.
+// (kPerLane per lane, for rows of at most 64 kPerLane minima): a binary
+// search on the key's bits, each step a count of the keys below by ballots,
+// ended by the first bound with exactly rank keys below it (about half of
+// the bits). No LDS: four radix passes over LDS histograms took 12.6 us for
+// 32 rows of 1,024 minima and 66 us for 32,768; this XXX.
 template <int kPerLane>
 __global__ __launch_bounds__(256) void probe_threshold_wave_kernel(const float* __restrict__ gm, int n_groups,
                                                                    int nrows, int rank, const float* __restrict__ rot,
@@ -767,7 +815,6 @@ __global__ __launch_bounds__(256) void probe_threshold_wave_kernel(const float* 
                                                                    float* __restrict__ thr,
                                                                    uint32_t* __restrict__ row_flag,
                                                                    uint32_t* __restrict__ nflag) {
-    __shared__ __align__(16) int hist_all[4][256];
     const int l = lane_id();
     const int row = static_cast<int>(blockIdx.x) * 4 + wave_id();
     if (row >= nrows) return;
@@ -775,48 +822,51 @@ __global__ __launch_bounds__(256) void probe_threshold_wave_kernel(const float* 
         row_flag[row] = 0u;
         if (row == 0) *nflag = 0u;
     }
-    int* hist = hist_all[wave_id()];
     const float* src = gm + static_cast<size_t>(row) * n_groups;
     uint32_t key[kPerLane];
 #pragma unroll
     for (int u = 0; u < kPerLane; ++u) {
         const int g = u * kWave + l;
-        key[u] = g < n_groups ? float_to_ordered(src[g]) : 0u;
+        key[u] = g < n_groups ? float_to_ordered(src[g]) : 0xFFFFFFFFu;
     }
-    uint32_t prefix = 0u, pmask = 0u;
-    int rem = rank;  // position (1-based, ascending) within the keys that share the prefix
-    for (int shift = 24; shift >= 0; shift -= 8) {
-        *reinterpret_cast<int4*>(&hist[4 * l]) = make_int4(0, 0, 0, 0);
-        wave_lds_sync();
+    // the largest t with fewer than rank keys below it is the rank-th
+    // smallest key: bit by bit below the keys' common prefix
+    uint32_t lo = 0xFFFFFFFFu, hi = 0u;
 #pragma unroll
-        for (int u = 0; u < kPerLane; ++u)
-            wave_hist_add(hist, u * kWave + l < n_groups && (key[u] & pmask) == prefix, (key[u] >> shift) & 255u);
-        wave_lds_sync();
-        const int4 h = *reinterpret_cast<const int4*>(&hist[4 * l]);
-        const int hv[4] = {h.x, h.y, h.z, h.w};
-        const int own = h.x + h.y + h.z + h.w;
-        const int incl = wave_inclusive_scan(own);
-        const int excl = incl - own;
-        // at least rem keys share the prefix, so exactly one lane holds the digit
-        const bool mine = excl < rem && incl >= rem;
-        int bin = 0, cum = 0;
-        if (mine) {
-            cum = excl;
-            int qd = 0;
-            while (qd < 3 && cum + hv[qd] < rem) {
-                cum += hv[qd];
-                ++qd;
+    for (int u = 0; u < kPerLane; ++u) {
+        const bool in = u * kWave + l < n_groups;
+        lo = key[u] < lo ? key[u] : lo;
+        hi = in && key[u] > hi ? key[u] : hi;
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        const uint32_t a = static_cast<uint32_t>(__shfl_xor(static_cast<int>(lo), o, kWave));
+        const uint32_t b = static_cast<uint32_t>(__shfl_xor(static_cast<int>(hi), o, kWave));
+        lo = a < lo ? a : lo;
+        hi = b > hi ? b : hi;
+    }
+    lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(lo)));
+    hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(hi)));
+    const int top = lo == hi ? -1 : 31 - __builtin_clz(lo ^ hi);
+    uint32_t prefix = top < 0 ? lo : top == 31 ? 0u : hi >> (top + 1) << (top + 1);
+    for (int bit = top; bit >= 0; --bit) {
+        const uint32_t t = prefix | (1u << bit);
+        int below = 0;
+#pragma unroll
+        for (int u = 0; u < kPerLane; ++u) below += __popcll(__ballot(key[u] < t));
+        if (below == rank) {  // the largest key below t
+            uint32_t m = 0u;
+#pragma unroll
+            for (int u = 0; u < kPerLane; ++u) m = key[u] < t && key[u] > m ? key[u] : m;
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) {
+                const uint32_t b = static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), o, kWave));
+                m = b > m ? b : m;
             }
-            bin = 4 * l + qd;
+            prefix = m;
+            break;
         }
-        const uint64_t who = __ballot(mine);
-        const int src_lane = who != 0ull ? __ffsll(static_cast<long long>(who)) - 1 : kWave - 1;
-        bin = __builtin_amdgcn_readlane(bin, src_lane);
-        cum = __builtin_amdgcn_readlane(cum, src_lane);
-        prefix |= static_cast<uint32_t>(bin) << shift;
-        rem -= cum;
-        pmask |= 255u << shift;
-        wave_lds_sync();  // the next pass clears hist
+        if (below < rank) prefix = t;
     }
     const float2 nq = row_norms_wave(rot + static_cast<size_t>(row) * kDim);
     if (l == 0) thr[row] = ordered_to_float(prefix) + 2.0f * probe_delta(nq.x, eq_weight * nq.y, cmax, ecmax);
@@ -844,7 +894,12 @@ __global__ __launch_bounds__(256) void probe_threshold_wave_kernel(const float* 
 // of its nsub sub-lists. Rows with more than max_n candidates (row_cand
 // 0xFFFFFFFF), a saturated value or a failed check (0xFFFFFFFE) are left to
 // the exact kernel.
+// kGroup sub-lists (64, or 512 where a row has more than 64: few rows, split
+// over every CU) form one index space at a time, so that a row's counts and
+// then its records are each about one round trip.
 constexpr int kRerankWaves = 2;
+constexpr int kRerankGroupMany = 512;
+template <int kGroup>
 __global__ __launch_bounds__(kRerankWaves * kWave) void probe_rerank_kernel(
     const float* __restrict__ rot, int nrows, const float* __restrict__ centroids, const float* __restrict__ norms,
     const uint4* __restrict__ rval, const uint32_t* __restrict__ rtile, const uint32_t* __restrict__ cnt,
@@ -853,7 +908,7 @@ __global__ __launch_bounds__(kRerankWaves * kWave) void probe_rerank_kernel(
     uint32_t* __restrict__ list, uint32_t* __restrict__ nflag, int list_cap) {
     extern __shared__ uint64_t smem_keys[];  // [kRerankWaves][max_n]
     __shared__ float qs[kRerankWaves][kDim];
-    __shared__ __align__(16) int hist_all[kRerankWaves][256];
+    __shared__ __align__(16) int hist_all[kRerankWaves][kGroup > 256 ? kGroup : 256];
     const int w = wave_id();
     const int l = lane_id();
     const int row = static_cast<int>(blockIdx.x) * kRerankWaves + w;
@@ -885,13 +940,25 @@ __global__ __launch_bounds__(kRerankWaves * kWave) void probe_rerank_kernel(
     int n = 0;
     uint32_t hmax = 0u;  // largest v's bits (>= 0x7BFF: saturated, inf or NaN)
     const uint32_t* c_row = cnt + static_cast<size_t>(row) * nsub;
-    int* pre = hist;  // [64] exclusive prefix of the sub-list counts
-    for (int s0 = 0; s0 < nsub; s0 += kWave) {
-        const int ns = nsub - s0 < kWave ? nsub - s0 : kWave;
-        const int mycnt = l < ns ? static_cast<int>(c_row[s0 + l]) : 0;
+    int* pre = hist;  // [kGroup] exclusive prefix of the sub-list counts
+    constexpr int kPer = kGroup / kWave;  // consecutive sub-lists of a lane
+    for (int s0 = 0; s0 < nsub; s0 += kGroup) {
+        const int ns = nsub - s0 < kGroup ? nsub - s0 : kGroup;
+        int lcnt[kPer];
+        int mycnt = 0;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            lcnt[u] = kPer * l + u < ns ? static_cast<int>(c_row[s0 + kPer * l + u]) : 0;
+            mycnt += lcnt[u];
+        }
         const int cincl = wave_inclusive_scan(mycnt);
         const int total = __builtin_amdgcn_readlane(cincl, kWave - 1);
-        pre[l] = cincl - mycnt;
+        int run = cincl - mycnt;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            pre[kPer * l + u] = run;
+            run += lcnt[u];
+        }
         wave_lds_sync();
         // record g of this group: tile, 8 value words, lane half of its sub-list
         struct Rec {
@@ -906,7 +973,7 @@ __global__ __launch_bounds__(kRerankWaves * kWave) void probe_rerank_kernel(
             const int gc = g < total ? g : 0;
             int sl = 0;
 #pragma unroll
-            for (int step = 32; step >= 1; step >>= 1)
+            for (int step = kGroup / 2; step >= 1; step >>= 1)
                 if (sl + step < ns && pre[sl + step] <= gc) sl += step;
             const size_t e = (static_cast<size_t>(row) * nsub + s0 + sl) * lane_cap + (gc - pre[sl]);
             r.tile = rtile[e];
@@ -1282,6 +1349,8 @@ ProbePlan plan_probe_mfma(int nrows, int64_t k, int nprobe, int num_cus) {
     p.tiles_per_split = (p.tiles_per_split + unit - 1) / unit * unit;
     p.splits = static_cast<int>((ntiles + p.tiles_per_split - 1) / p.tiles_per_split);
     p.lane_cap = kProbeLaneCap;
+    // one row block that its rows do not fill: waves share the rows there are
+    p.wave_share = nrows <= kRowsPerBlock / 8 ? 8 : nrows <= kRowsPerBlock / 2 ? 2 : 1;
     const int n_groups = (p.n_sampled + p.group_tiles - 1) / p.group_tiles;
     p.usable = n_groups >= nprobe && n_groups <= kMaxGroups && nprobe <= 1024 && 2 * p.splits <= kMaxSublists;
     return p;
@@ -1311,14 +1380,21 @@ hipError_t launch_probe_mfma(hipStream_t s, const ProbePlan& p, const float* rot
                 hipLaunchKernelGGL((probe_mfma_f32_kernel<0, 1>), grid, dim3(kF32Waves * kWave), 0, s, rot, nrows,
                                    centroids, nhalf, k, p.tiles_per_split, p.sample_stride, gm, thr, nullptr, nullptr,
                                    cnt, p.lane_cap, row_flag, p.row_blocks, p.splits);
-        } else if (p.group_tiles == kGroupTiles) {
-            hipLaunchKernelGGL((probe_mfma_kernel<0, kGroupTiles>), grid, dim3(kProbeWaves * kWave), 0, s, rot, nrows,
-                               cbf, nhalf, k, p.tiles_per_split, p.sample_stride, gm, thr, nullptr, nullptr, nullptr,
-                               cnt, p.lane_cap, row_flag, nullptr, cmax, ecmax, p.row_blocks, p.splits);
         } else {
-            hipLaunchKernelGGL((probe_mfma_kernel<0, 1>), grid, dim3(kProbeWaves * kWave), 0, s, rot, nrows, cbf,
-                               nhalf, k, p.tiles_per_split, p.sample_stride, gm, thr, nullptr, nullptr, nullptr, cnt,
-                               p.lane_cap, row_flag, nullptr, cmax, ecmax, p.row_blocks, p.splits);
+            auto pass = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, grid, dim3(kProbeWaves * kWave), 0, s, rot, nrows, cbf, nhalf, k,
+                                   p.tiles_per_split, p.sample_stride, gm, thr, nullptr, nullptr, nullptr, cnt,
+                                   p.lane_cap, row_flag, nullptr, cmax, ecmax, p.row_blocks, p.splits);
+            };
+            if (p.group_tiles == kGroupTiles) {
+                if (p.wave_share == 8) pass(probe_mfma_kernel<0, kGroupTiles, 8>);
+                else if (p.wave_share == 2) pass(probe_mfma_kernel<0, kGroupTiles, 2>);
+                else pass(probe_mfma_kernel<0, kGroupTiles, 1>);
+            } else {
+                if (p.wave_share == 8) pass(probe_mfma_kernel<0, 1, 8>);
+                else if (p.wave_share == 2) pass(probe_mfma_kernel<0, 1, 2>);
+                else pass(probe_mfma_kernel<0, 1, 1>);
+            }
         }
         if ((e = hipGetLastError()) != hipSuccess) return e;
         const dim3 wgrid((nrows + 3) / 4);
@@ -1341,10 +1417,16 @@ hipError_t launch_probe_mfma(hipStream_t s, const ProbePlan& p, const float* rot
             hipLaunchKernelGGL(probe_mfma_f32_kernel<1>, grid, dim3(kF32Waves * kWave), 0, s, rot, nrows, centroids,
                                nhalf, k, p.tiles_per_split, 1, gm, thr, rv, rtile, cnt, p.lane_cap, row_flag,
                                p.row_blocks, p.splits);
-        else
-            hipLaunchKernelGGL(probe_mfma_kernel<1>, grid, dim3(kProbeWaves * kWave), 0, s, rot, nrows, cbf, nhalf, k,
-                               p.tiles_per_split, 1, gm, thr, nullptr, rv, rtile, cnt, p.lane_cap, row_flag, nullptr,
-                               cmax, ecmax, p.row_blocks, p.splits);
+        else {
+            auto pass = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, grid, dim3(kProbeWaves * kWave), 0, s, rot, nrows, cbf, nhalf, k,
+                                   p.tiles_per_split, 1, gm, thr, nullptr, rv, rtile, cnt, p.lane_cap, row_flag, nullptr,
+                                   cmax, ecmax, p.row_blocks, p.splits);
+            };
+            if (p.wave_share == 8) pass(probe_mfma_kernel<1, kGroupTiles, 8>);
+            else if (p.wave_share == 2) pass(probe_mfma_kernel<1, kGroupTiles, 2>);
+            else pass(probe_mfma_kernel<1, kGroupTiles, 1>);
+        }
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (part < 0 || part == 2) {
@@ -1353,10 +1435,17 @@ hipError_t launch_probe_mfma(hipStream_t s, const ProbePlan& p, const float* rot
         // takes sets the rerank's occupancy (16 waves per CU at 1024)
         int max_n = 1024;
         while (max_n < 8 * nprobe && max_n < kProbeMaxCandidates) max_n *= 2;
-        hipLaunchKernelGGL(probe_rerank_kernel, dim3((nrows + kRerankWaves - 1) / kRerankWaves),
-                           dim3(kRerankWaves * kWave), static_cast<size_t>(kRerankWaves) * max_n * 8, s, rot, nrows,
-                           centroids, norms, rv, rtile, cnt, p.lane_cap, 2 * p.splits, max_n, nprobe,
-                           p.u_rank >= nprobe, cmax, ec, eqw, row_flag, row_cand, labels, fb.list, fb.nflag, fb.list_cap);
+        const int nsub = 2 * p.splits;
+        auto rerank = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((nrows + kRerankWaves - 1) / kRerankWaves), dim3(kRerankWaves * kWave),
+                               static_cast<size_t>(kRerankWaves) * max_n * 8, s, rot, nrows, centroids, norms, rv, rtile,
+                               cnt, p.lane_cap, nsub, max_n, nprobe, p.u_rank >= nprobe, cmax, ec, eqw, row_flag,
+                               row_cand, labels, fb.list, fb.nflag, fb.list_cap);
+        };
+        if (nsub <= kWave)
+            rerank(probe_rerank_kernel<kWave>);
+        else
+            rerank(probe_rerank_kernel<kRerankGroupMany>);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         // rows that overflowed or failed the check: exact recomputation
         e = launch_probe_exact_flagged(s, rot, nrows, centroids, norms, k, nprobe, row_flag, labels, fb, true);
