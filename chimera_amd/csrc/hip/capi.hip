@@ -5,11 +5,13 @@
 #include "kernels.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -108,16 +110,26 @@ struct WorkspaceShape {
     int blog;      // documents per candidate bucket = 2^blog
 };
 
-// Bytes of a workspace of this shape (arrays at 256-byte boundaries); with a
-// base, also the pointers into it.
-size_t carve_workspace(const WorkspaceShape& sh, unsigned char* base, Workspace* w) {
+// Arrays laid out one after the other at 256-byte boundaries: without a base
+// their total size, with one the pointers too. One allocation for many
+// arrays: a hipMalloc and its hipFree cost 0.1 ms and more whatever the size,
+// and an index build made 49 of each (6.8 ms).
+struct Carver {
+    unsigned char* base = nullptr;
     size_t off = 0;
-    auto take = [&](auto*& p, size_t count) {
-        using T = std::remove_reference_t<decltype(*p)>;
+    template <typename T>
+    void operator()(T*& p, size_t count) {
         off = (off + 255) / 256 * 256;
         if (base) p = reinterpret_cast<T*>(base + off);
         off += std::max<size_t>(count, 1) * sizeof(T);
-    };
+    }
+    size_t bytes() const { return (off + 255) / 256 * 256; }
+};
+
+// Bytes of a workspace of this shape; with a base, also the pointers into it.
+size_t carve_workspace(const WorkspaceShape& sh, unsigned char* base, Workspace* w) {
+    Carver take;
+    take.base = base;
     Workspace tmp;
     Workspace& x = w ? *w : tmp;
     const size_t B = sh.batch, QS = sh.qs;
@@ -150,14 +162,22 @@ size_t carve_workspace(const WorkspaceShape& sh, unsigned char* base, Workspace*
     take(x.err, 1);
     if (sh.staging) take(x.out_counts, B);
     x.qs = static_cast<int>(QS);
-    return (off + 255) / 256 * 256;
+    return take.bytes();
 }
+
+struct DevBlock {
+    void* ptr;
+    size_t bytes;
+};
 
 struct chimera_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
-    std::vector<void*> index_allocs;
-    std::vector<void*> ws_allocs;
+    std::vector<DevBlock> index_allocs;
+    std::vector<DevBlock> ws_allocs;
+    // blocks of the index that a build or upload replaces, for its own
+    // allocations; the rest is freed when it ends
+    std::vector<DevBlock> spare;
     uint64_t bytes = 0;
 
     bool has_index = false;
@@ -242,33 +262,81 @@ struct chimera_ctx {
 
 namespace {
 
-template <typename T>
-int dev_alloc(chimera_ctx* c, std::vector<void*>& list, T** p, size_t count, const char* what) {
-    *p = nullptr;
-    if (count == 0) count = 1;
-    void* ptr = nullptr;
-    const hipError_t e = hipMalloc(&ptr, count * sizeof(T));
-    if (e != hipSuccess) {
-        return fail(CHIMERA_ERR_HIP, std::string("hipMalloc of ") + what + " (" + std::to_string(count * sizeof(T)) +
-                                         " bytes) failed: " + hipGetErrorString(e));
-    }
-    list.push_back(ptr);
-    c->bytes += count * sizeof(T);
-    *p = static_cast<T*>(ptr);
-    return CHIMERA_OK;
-}
-
-void free_list(std::vector<void*>& list) {
-    for (void* p : list) (void)hipFree(p);
+void free_list(std::vector<DevBlock>& list) {
+    for (const DevBlock& b : list) (void)hipFree(b.ptr);
     list.clear();
 }
 
-void release_index(chimera_ctx* c) {
+template <typename T>
+int dev_alloc(chimera_ctx* c, std::vector<DevBlock>& list, T** p, size_t count, const char* what) {
+    *p = nullptr;
+    if (count == 0) count = 1;
+    const size_t bytes = count * sizeof(T);
+    DevBlock block{nullptr, bytes};
+    // the smallest spare block that holds it without wasting a quarter
+    auto fit = c->spare.end();
+    for (auto it = c->spare.begin(); it != c->spare.end(); ++it)
+        if (it->bytes >= bytes && it->bytes - bytes <= bytes / 4 && (fit == c->spare.end() || it->bytes < fit->bytes)) fit = it;
+    if (fit != c->spare.end()) {
+        block = *fit;
+        c->spare.erase(fit);
+    } else {
+        hipError_t e = hipMalloc(&block.ptr, bytes);
+        if (e != hipSuccess && !c->spare.empty()) {
+            (void)hipGetLastError();
+            free_list(c->spare);
+            e = hipMalloc(&block.ptr, bytes);
+        }
+        if (e != hipSuccess) {
+            return fail(CHIMERA_ERR_HIP, std::string("hipMalloc of ") + what + " (" + std::to_string(bytes) +
+                                             " bytes) failed: " + hipGetErrorString(e));
+        }
+    }
+    list.push_back(block);
+    c->bytes += block.bytes;
+    *p = static_cast<T*>(block.ptr);
+    return CHIMERA_OK;
+}
+
+// Frees one block of `list`.
+void dev_free(chimera_ctx* c, std::vector<DevBlock>& list, void* ptr) {
+    for (auto it = list.begin(); it != list.end(); ++it) {
+        if (it->ptr != ptr) continue;
+        c->bytes -= it->bytes;
+        list.erase(it);
+        break;
+    }
+    (void)hipFree(ptr);
+}
+
+// One allocation of the context's `list` for the arrays that `lay` takes.
+template <typename Lay>
+int dev_carve(chimera_ctx* c, std::vector<DevBlock>& list, const char* what, Lay&& lay) {
+    Carver sizes;
+    lay(sizes);
+    Carver arrays;
+    CK(dev_alloc(c, list, &arrays.base, sizes.bytes(), what));
+    lay(arrays);
+    return CHIMERA_OK;
+}
+
+// Empties the context; with `reuse`, its blocks stay as spares (a Rebuild
+// ends that). Freeing and allocating an index's gigabytes anew is cheap only
+// while the driver has cleared memory in stock: builds and downloads of 0.88M
+// tokens one after the other took 15 ms each at first and 180 ms once it was
+// used up; with the blocks reused 11 ms.
+void release_index(chimera_ctx* c, bool reuse = false) {
     if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
     if (c->graph) (void)hipGraphDestroy(c->graph);
     c->graph_exec = nullptr;
     c->graph = nullptr;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
+    if (reuse) {
+        c->spare.insert(c->spare.end(), c->index_allocs.begin(), c->index_allocs.end());
+        c->spare.insert(c->spare.end(), c->ws_allocs.begin(), c->ws_allocs.end());
+        c->index_allocs.clear();
+        c->ws_allocs.clear();
+    }
     free_list(c->ws_allocs);
     free_list(c->index_allocs);
     c->bytes = 0;
@@ -284,8 +352,17 @@ void release_index(chimera_ctx* c) {
     c->cnh = nullptr;
     c->p_err = nullptr;
     c->p_ncand = nullptr;
+    c->p_rval = nullptr;
     c->p_xfb = ExactFallback{};
 }
+
+// Scope of a build or upload into a context: the spares it did not take are
+// freed at its end.
+struct Rebuild {
+    chimera_ctx* c;
+    explicit Rebuild(chimera_ctx* ctx) : c(ctx) { release_index(c, true); }
+    ~Rebuild() { free_list(c->spare); }
+};
 
 int set_device(chimera_ctx* c) {
     CK_HIP(hipSetDevice(c->device), "hipSetDevice");
@@ -369,6 +446,10 @@ int collect_stage_times(chimera_ctx* c) {
 struct TempBuffers {
     hipStream_t stream = nullptr;
     std::vector<void*> ptrs;
+    // memory of the context that nothing else uses meanwhile: carve() takes
+    // from it what fits
+    unsigned char* region = nullptr;
+    size_t region_bytes = 0;
     ~TempBuffers() {
         if (stream) (void)hipStreamSynchronize(stream);
         for (void* p : ptrs) (void)hipFree(p);
@@ -388,12 +469,26 @@ struct TempBuffers {
         *p = static_cast<T*>(ptr);
         return CHIMERA_OK;
     }
-    void release(void* p) {
-        auto it = std::find(ptrs.begin(), ptrs.end(), p);
-        if (it == ptrs.end()) return;
+    // one allocation for the arrays that `lay` takes
+    template <typename Lay>
+    int carve(const char* what, Lay&& lay) {
+        Carver sizes;
+        lay(sizes);
+        Carver arrays;
+        if (sizes.bytes() <= region_bytes) {
+            arrays.base = region;
+            region += sizes.bytes();
+            region_bytes -= sizes.bytes();
+        } else {
+            CK(alloc(&arrays.base, sizes.bytes(), what));
+        }
+        lay(arrays);
+        return CHIMERA_OK;
+    }
+    void release() {
         if (stream) (void)hipStreamSynchronize(stream);
-        (void)hipFree(p);
-        ptrs.erase(it);
+        for (void* p : ptrs) (void)hipFree(p);
+        ptrs.clear();
     }
 };
 
@@ -656,6 +751,105 @@ int run_pipeline(chimera_ctx* c, const Workspace& w, const float* d_queries, int
     return run_back(c, w, s, 0, nq, k, d_ids, d_scores, d_counts, d_status);
 }
 
+// Grows the pinned staging buffer to hold `host` bytes.
+int ensure_stage(chimera_ctx* c, size_t host) {
+    if (host <= c->h_stage_bytes) return CHIMERA_OK;
+    CK_HIP(hipStreamSynchronize(c->stream), "synchronising before staging growth");
+    if (c->h_stage) (void)hipHostFree(c->h_stage);
+    c->h_stage = nullptr;
+    c->d_stage = nullptr;
+    c->h_stage_bytes = 0;
+    const size_t bytes = (host + 4095) / 4096 * 4096;
+    void* p = nullptr;
+    CK_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault), "pinned staging buffer");
+    c->h_stage = static_cast<unsigned char*>(p);
+    c->h_stage_bytes = bytes;
+    void* dp = nullptr;
+    c->d_stage = hipHostGetDevicePointer(&dp, p, 0) == hipSuccess ? static_cast<unsigned char*>(dp) : nullptr;
+    return CHIMERA_OK;
+}
+
+// Downloads of large arrays into pageable memory. The runtime's own copy runs
+// at the rate at which one thread takes the destination's page faults and
+// copies (0.12 GB of a 0.88M-token index: 16 ms); here DMA copies fill a ring
+// of pinned slots while a thread per slot copies out of it (XXX ms).
+constexpr size_t kSlotBytes = size_t{2} << 20;
+constexpr int kCopyThreads = 8;
+
+struct HostCopy {
+    unsigned char* dst;
+    const unsigned char* src;  // device
+    size_t bytes;
+};
+
+int download_arrays(chimera_ctx* c, const std::vector<HostCopy>& arrays) {
+    std::vector<HostCopy> chunks;
+    for (const HostCopy& a : arrays)
+        for (size_t o = 0; o < a.bytes; o += kSlotBytes)
+            chunks.push_back({a.dst + o, a.src + o, std::min(kSlotBytes, a.bytes - o)});
+    const size_t n = chunks.size();
+    hipEvent_t landed[kCopyThreads] = {};
+    std::atomic<int64_t> issued[kCopyThreads];  // copies queued into the slot, -1: no more
+    std::atomic<int64_t> taken[kCopyThreads];   // copies taken out of it
+    std::atomic<int> error{hipSuccess};
+    std::vector<std::thread> threads;
+    for (int t = 0; t < kCopyThreads; ++t) {
+        issued[t] = 0;
+        taken[t] = 0;
+    }
+    auto worker = [&](int t) {
+        (void)hipSetDevice(c->device);
+        for (int64_t k = 0;; ++k) {
+            const size_t i = static_cast<size_t>(k) * kCopyThreads + static_cast<size_t>(t);
+            if (i >= n) return;
+            int64_t q;
+            while ((q = issued[t].load(std::memory_order_acquire)) >= 0 && q <= k) std::this_thread::yield();
+            if (q < 0) return;
+            const hipError_t e = hipEventSynchronize(landed[t]);
+            if (e != hipSuccess) error = e;
+            std::memcpy(chunks[i].dst, c->h_stage + static_cast<size_t>(t) * kSlotBytes, chunks[i].bytes);
+            taken[t].store(k + 1, std::memory_order_release);
+        }
+    };
+    hipError_t e = hipSuccess;
+    for (int t = 0; t < kCopyThreads && e == hipSuccess; ++t) e = hipEventCreateWithFlags(&landed[t], hipEventDisableTiming);
+    size_t done = 0;  // chunks in the workers' hands
+    if (e == hipSuccess) {
+        try {
+            threads.reserve(kCopyThreads);
+            for (int t = 0; t < kCopyThreads; ++t) threads.emplace_back(worker, t);
+        } catch (const std::exception&) {
+            // fewer threads than slots: the loop below stops at the first
+            // slot without one, and the rest is copied directly
+        }
+        for (; done < n && e == hipSuccess; ++done) {
+            const int t = static_cast<int>(done % kCopyThreads);
+            if (static_cast<size_t>(t) >= threads.size()) break;
+            const int64_t k = static_cast<int64_t>(done / kCopyThreads);
+            while (taken[t].load(std::memory_order_acquire) < k) std::this_thread::yield();
+            e = hipMemcpyAsync(c->h_stage + static_cast<size_t>(t) * kSlotBytes, chunks[done].src, chunks[done].bytes,
+                               hipMemcpyDeviceToHost, c->stream);
+            if (e == hipSuccess) e = hipEventRecord(landed[t], c->stream);
+            if (e != hipSuccess) break;
+            issued[t].store(k + 1, std::memory_order_release);
+        }
+    }
+    // the workers finish what was queued, then leave
+    for (int t = 0; t < static_cast<int>(threads.size()); ++t) {
+        const int64_t last = issued[t].load();
+        while (taken[t].load(std::memory_order_acquire) < last) std::this_thread::yield();
+        issued[t].store(-1, std::memory_order_release);
+    }
+    for (std::thread& t : threads) t.join();
+    for (hipEvent_t ev : landed)
+        if (ev) (void)hipEventDestroy(ev);
+    for (; done < n && e == hipSuccess; ++done)
+        e = hipMemcpy(chunks[done].dst, chunks[done].src, chunks[done].bytes, hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = static_cast<hipError_t>(error.load());
+    CK_HIP(e, "index download");
+    return CHIMERA_OK;
+}
+
 // Host batches of up to this many bytes of queries (eight of 128 dimensions)
 // skip the copies, each a launch of its own around a search of a few
 // hundred us. 37 queries (0.45 MB) took the same either way (541 and 545 us):
@@ -673,10 +867,7 @@ int ensure_out(chimera_ctx* c, int32_t nq, int32_t k, size_t host_bytes, bool di
         CK_HIP(hipStreamSynchronize(c->stream), "synchronising before output growth");
         // the region lives with the workspace; the old one leaves the list
         if (c->w_out) {
-            auto it = std::find(c->ws_allocs.begin(), c->ws_allocs.end(), static_cast<void*>(c->w_out));
-            if (it != c->ws_allocs.end()) c->ws_allocs.erase(it);
-            (void)hipFree(c->w_out);
-            c->bytes -= c->w_out_bytes;
+            dev_free(c, c->ws_allocs, c->w_out);
             c->w_out = nullptr;
             c->w_out_bytes = 0;
         }
@@ -684,21 +875,7 @@ int ensure_out(chimera_ctx* c, int32_t nq, int32_t k, size_t host_bytes, bool di
         CK(dev_alloc(c, c->ws_allocs, &c->w_out, bytes, "search results"));
         c->w_out_bytes = bytes;
     }
-    const size_t host = std::max(used, host_bytes);
-    if (host > c->h_stage_bytes) {
-        CK_HIP(hipStreamSynchronize(c->stream), "synchronising before staging growth");
-        if (c->h_stage) (void)hipHostFree(c->h_stage);
-        c->h_stage = nullptr;
-        c->d_stage = nullptr;
-        c->h_stage_bytes = 0;
-        const size_t bytes = (host + 4095) / 4096 * 4096;
-        void* p = nullptr;
-        CK_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault), "pinned staging buffer");
-        c->h_stage = static_cast<unsigned char*>(p);
-        c->h_stage_bytes = bytes;
-        void* dp = nullptr;
-        c->d_stage = hipHostGetDevicePointer(&dp, p, 0) == hipSuccess ? static_cast<unsigned char*>(dp) : nullptr;
-    }
+    CK(ensure_stage(c, std::max(used, host_bytes)));
     unsigned char* base = direct && c->d_stage ? c->d_stage : c->w_out;
     c->w_out_ids = reinterpret_cast<int64_t*>(base);
     c->w_out_scores = reinterpret_cast<float*>(base + m * 8);
@@ -708,6 +885,32 @@ int ensure_out(chimera_ctx* c, int32_t nq, int32_t k, size_t host_bytes, bool di
     return CHIMERA_OK;
 }
 
+
+// The matrix-core probe's buffers for batches of up to max_batch queries, once
+// per index.
+int alloc_probe(chimera_ctx* c, const ProbePlan& plan, int32_t max_batch) {
+    if (c->p_rval) return CHIMERA_OK;
+    const size_t rows = static_cast<size_t>(max_batch) * kQ;
+    const size_t sub_rows = probe_sublist_rows(max_batch * kQ, c->num_cus);
+    const size_t nrec = sub_rows * 2 * static_cast<size_t>(plan.lane_cap);
+    c->p_xfb.list_cap = kExactFallbackRows;
+    CK(dev_carve(c, c->index_allocs, "probe buffers", [&](Carver& take) {
+        take(c->cbf, static_cast<size_t>(c->n_clusters) * kDim);
+        take(c->cnh, static_cast<size_t>(c->n_clusters));
+        take(c->p_err, 1);
+        take(c->p_gm, static_cast<size_t>(plan.n_sampled) * rows);
+        take(c->p_thr, rows);
+        take(c->p_rval, nrec * 8);
+        take(c->p_rtile, nrec);
+        take(c->p_cnt, sub_rows * 2);
+        take(c->p_flag, rows);
+        take(c->p_ncand, rows);
+        take(c->p_xfb.list, kExactFallbackRows);
+        take(c->p_xfb.nflag, 1);
+        take(c->p_xfb.partial, static_cast<size_t>(kExactFallbackRows) * kExactPartialKeys);
+    }));
+    return CHIMERA_OK;
+}
 
 // Search-side state shared by index upload and device build: centroid norms
 // bound, matrix-core probe buffers, candidate bounds and the workspace. The
@@ -729,9 +932,7 @@ int finish_setup(chimera_ctx* c, const chimera_search_options& o, int32_t max_ba
         const ProbePlan plan = plan_probe_mfma(max_batch * kQ, c->n_clusters, opt->nprobe, c->num_cus);
         if (plan.usable) {
             const size_t rows = static_cast<size_t>(max_batch) * kQ;
-            CK(dev_alloc(c, c->index_allocs, &c->cbf, static_cast<size_t>(c->n_clusters) * kDim, "bf16 centroids"));
-            CK(dev_alloc(c, c->index_allocs, &c->cnh, static_cast<size_t>(c->n_clusters), "probe initial values"));
-            CK(dev_alloc(c, c->index_allocs, &c->p_err, 1, "centroid rounding bound"));
+            CK(alloc_probe(c, plan, max_batch));
             CK_HIP(launch_probe_centroids(c->stream, c->centroids, c->norms, c->n_clusters, c->cbf, c->cnh, c->p_err),
                    "bf16 centroids");
             uint32_t eb = 0;
@@ -741,21 +942,7 @@ int finish_setup(chimera_ctx* c, const chimera_search_options& o, int32_t max_ba
             std::memcpy(&ef, &eb, sizeof(ef));
             // the fp32 sum of 128 squares is within 1e-5 of |c - c_b|^2
             c->ecmax = static_cast<float>(static_cast<double>(ef) * (1.0 + 1e-4));
-            CK(dev_alloc(c, c->index_allocs, &c->p_gm, static_cast<size_t>(plan.n_sampled) * rows, "probe tile minima"));
-            CK(dev_alloc(c, c->index_allocs, &c->p_thr, rows, "probe thresholds"));
-            const size_t sub_rows = probe_sublist_rows(max_batch * kQ, c->num_cus);
-            const size_t nrec = sub_rows * 2 * static_cast<size_t>(plan.lane_cap);
-            CK(dev_alloc(c, c->index_allocs, &c->p_rval, nrec * 8, "probe records"));
-            CK(dev_alloc(c, c->index_allocs, &c->p_rtile, nrec, "probe record tiles"));
-            CK(dev_alloc(c, c->index_allocs, &c->p_cnt, sub_rows * 2, "probe counts"));
-            CK(dev_alloc(c, c->index_allocs, &c->p_flag, rows, "probe flags"));
-            CK(dev_alloc(c, c->index_allocs, &c->p_ncand, rows, "probe candidate counts"));
             CK_HIP(launch_fill_u32(c->stream, c->p_ncand, static_cast<int64_t>(rows), 0u), "probe candidate counts");
-            c->p_xfb.list_cap = kExactFallbackRows;
-            CK(dev_alloc(c, c->index_allocs, &c->p_xfb.list, kExactFallbackRows, "flagged probe rows"));
-            CK(dev_alloc(c, c->index_allocs, &c->p_xfb.nflag, 1, "flagged probe row count"));
-            CK(dev_alloc(c, c->index_allocs, &c->p_xfb.partial,
-                         static_cast<size_t>(kExactFallbackRows) * kExactPartialKeys, "flagged probe row keys"));
             c->probe_mfma_ready = true;
         }
     }
@@ -804,6 +991,10 @@ int finish_setup(chimera_ctx* c, const chimera_search_options& o, int32_t max_ba
 }
 
 
+// Rows per assignment launch: one row block for every CU twice over on 256
+// CUs, so that the candidate buffer (2 KB a row) stays at 0.5 GB.
+constexpr int64_t kAssignBatch = int64_t{1} << 18;
+
 // Index build on the device (build_index.cu:394-501 with the CAGRA
 // assignment replaced by the exact matrix-core nearest-centroid search).
 int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t dim_, const int32_t* doc_lens,
@@ -840,7 +1031,7 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
     CK(validate_options(*opt, static_cast<int64_t>(k_)));
     if (max_batch <= 0) return fail(CHIMERA_ERR_INVALID_ARGUMENT, "max_batch must be positive");
     CK(set_device(c));
-    release_index(c);
+    const Rebuild rebuild(c);
     const CandShape shape = cand_shape(static_cast<int64_t>(m_), static_cast<int64_t>(n_), static_cast<int64_t>(k_),
                                        opt->nprobe);
     CK_HIP(configure_kernels(cand_buckets(static_cast<int64_t>(m_), shape.blog), opt->nprobe, opt->k_refine,
@@ -864,21 +1055,48 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
     const int ex_bits = static_cast<int>(ex_bits_);
     const size_t width = static_cast<size_t>(1 + ex_bits);
     hipStream_t s = c->stream;
-    TempBuffers tmp;
+    // the build's own buffers: labels through the whole build, then those of
+    // the assignment and those of the sort, in the probe's record area where
+    // they fit (no search runs meanwhile)
+    TempBuffers keep, tmp;
+    keep.stream = s;
     tmp.stream = s;
+    {
+        const ProbePlan plan = plan_probe_mfma(max_batch * kQ, c->n_clusters, opt->nprobe, c->num_cus);
+        if (plan.usable) {
+            CK(alloc_probe(c, plan, max_batch));
+            keep.region = reinterpret_cast<unsigned char*>(c->p_rval);
+            keep.region_bytes = probe_sublist_rows(max_batch * kQ, c->num_cus) * 2 * static_cast<size_t>(plan.lane_cap) * 32;
+        }
+    }
 
-    CK(upload(c, &c->doc_ptrs, ptrs.data(), m_ + 1, "doc_ptrs"));
-    CK(upload(c, &c->flips, flips, 4 * kDim / 8, "rotator flips"));
-    CK(dev_alloc(c, c->index_allocs, &c->codes_tok, (n + kRefinePadTokens) * kCodeBytes, "token-order codes"));
-    CK(dev_alloc(c, c->index_allocs, &c->f1_tok, n + kRefinePadTokens, "token-order factors"));
+    CK(dev_carve(c, c->index_allocs, "token-order index arrays", [&](Carver& take) {
+        take(c->doc_ptrs, m_ + 1);
+        take(c->flips, 4 * kDim / 8);
+        take(c->codes_tok, (n + kRefinePadTokens) * kCodeBytes);
+        take(c->f1_tok, n + kRefinePadTokens);
+        take(c->full_codes, (n + kFullbitPadTokens) * 16 * width);
+        take(c->full_factors, n + kFullbitPadTokens);
+        take(c->centroids, K * kDim);
+        take(c->norms, K);
+    }));
+    CK_HIP(hipMemcpy(c->doc_ptrs, ptrs.data(), (m_ + 1) * sizeof(int32_t), hipMemcpyHostToDevice), "doc_ptrs");
+    CK_HIP(hipMemcpy(c->flips, flips, 4 * kDim / 8, hipMemcpyHostToDevice), "rotator flips");
     CK_HIP(hipMemsetAsync(c->codes_tok + n * kCodeBytes, 0, kRefinePadTokens * kCodeBytes, s), "code padding");
     CK_HIP(hipMemsetAsync(c->f1_tok + n, 0, kRefinePadTokens * sizeof(float), s), "factor padding");
-    CK(dev_alloc(c, c->index_allocs, &c->full_codes, (n + kFullbitPadTokens) * 16 * width, "full codes"));
-    CK(dev_alloc(c, c->index_allocs, &c->full_factors, n + kFullbitPadTokens, "full factors"));
     CK_HIP(hipMemsetAsync(c->full_codes + n * 16 * width, 0, kFullbitPadTokens * 16 * width, s), "full code padding");
     CK_HIP(hipMemsetAsync(c->full_factors + n, 0, kFullbitPadTokens * sizeof(float), s), "full factor padding");
-    uint32_t* status = nullptr;
-    CK(tmp.alloc(&status, 1, "build status"));
+    uint32_t *status = nullptr, *labels = nullptr;
+    int64_t* d_ids = nullptr;
+    CK(keep.carve("build labels", [&](Carver& take) {
+        take(status, 1);
+        take(labels, n);
+        take(d_ids, K);
+    }));
+    unsigned char* const region = keep.region;
+    const size_t region_bytes = keep.region_bytes;
+    tmp.region = region;
+    tmp.region_bytes = region_bytes;
     CK_HIP(launch_fill_u32(s, status, 1, 0u), "clearing build status");
 
     // encode every token (build_index.cu:258-303)
@@ -887,28 +1105,40 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
            "token encoding");
 
     // rotated centroids (build_index.cu:221-238)
-    int64_t* d_ids = nullptr;
-    CK(tmp.alloc(&d_ids, K, "centroid ids"));
     CK_HIP(hipMemcpyAsync(d_ids, centroid_ids, K * sizeof(int64_t), hipMemcpyHostToDevice, s), "centroid ids");
-    CK(dev_alloc(c, c->index_allocs, &c->centroids, K * kDim, "centroids"));
-    CK(dev_alloc(c, c->index_allocs, &c->norms, K, "centroid norms"));
     CK_HIP(launch_gather_rows(s, d_emb, dim, d_ids, c->n_clusters, c->flips, true, c->centroids), "centroid rotation");
     CK_HIP(launch_centroid_norms(s, c->centroids, c->n_clusters, c->norms), "centroid norms");
 
     // nearest-centroid assignment in the input space (build_index.cu:186-219)
-    uint32_t* labels = nullptr;
-    CK(tmp.alloc(&labels, n, "assignments"));
     {
         float* cu = nullptr;
         float* nu = nullptr;
         float* nhu = nullptr;
         uint16_t* cbu = nullptr;
         uint32_t* ebu = nullptr;
-        CK(tmp.alloc(&cu, K * kDim, "assignment centroids"));
-        CK(tmp.alloc(&nu, K, "assignment centroid norms"));
-        CK(tmp.alloc(&nhu, K, "assignment probe initial values"));
-        CK(tmp.alloc(&cbu, K * kDim, "assignment bf16 centroids"));
-        CK(tmp.alloc(&ebu, 1, "assignment centroid rounding bound"));
+        const int64_t batch = std::min<int64_t>(c->n, kAssignBatch);
+        const ProbePlan full_plan = plan_assign_top1(static_cast<int>(batch), c->n_clusters, c->num_cus);
+        const size_t sub_rows = probe_sublist_rows(static_cast<int>(batch), c->num_cus);
+        uint32_t *ukey = nullptr, *cnt = nullptr, *flag = nullptr;
+        uint2* buf = nullptr;
+        float* padded = nullptr;
+        ExactFallback xfb;
+        xfb.list_cap = kExactFallbackRows;
+        CK(tmp.carve("assignment buffers", [&](Carver& take) {
+            take(cu, K * kDim);
+            take(nu, K);
+            take(nhu, K);
+            take(cbu, K * kDim);
+            take(ebu, 1);
+            take(ukey, static_cast<size_t>(batch));
+            take(cnt, sub_rows * 2);
+            take(flag, static_cast<size_t>(batch));
+            take(buf, sub_rows * 2 * static_cast<size_t>(full_plan.lane_cap));
+            take(xfb.list, static_cast<size_t>(kExactFallbackRows));
+            take(xfb.nflag, 1);
+            take(xfb.partial, static_cast<size_t>(kExactFallbackRows) * kExactPartialKeys);
+            if (dim < kDim) take(padded, static_cast<size_t>(batch) * kDim);
+        }));
         CK_HIP(launch_gather_rows(s, d_emb, dim, d_ids, c->n_clusters, nullptr, false, cu), "centroid gather");
         CK_HIP(launch_centroid_norms(s, cu, c->n_clusters, nu), "centroid norms");
         CK_HIP(launch_probe_centroids(s, cu, nu, c->n_clusters, cbu, nhu, ebu), "bf16 centroids");
@@ -923,23 +1153,6 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
         float ef = 0.0f;
         std::memcpy(&ef, &eb, sizeof(ef));
         const float ecmax = static_cast<float>(static_cast<double>(ef) * (1.0 + 1e-4));
-        const int64_t batch = std::min<int64_t>(c->n, int64_t{1} << 20);
-        const ProbePlan full_plan = plan_assign_top1(static_cast<int>(batch), c->n_clusters, c->num_cus);
-        uint32_t *ukey = nullptr, *cnt = nullptr, *flag = nullptr;
-        uint2* buf = nullptr;
-        CK(tmp.alloc(&ukey, static_cast<size_t>(batch), "assignment keys"));
-        const size_t sub_rows = probe_sublist_rows(static_cast<int>(batch), c->num_cus);
-        CK(tmp.alloc(&cnt, sub_rows * 2, "assignment counts"));
-        CK(tmp.alloc(&flag, static_cast<size_t>(batch), "assignment flags"));
-        CK(tmp.alloc(&buf, sub_rows * 2 * static_cast<size_t>(full_plan.lane_cap), "assignment candidates"));
-        ExactFallback xfb;
-        xfb.list_cap = kExactFallbackRows;
-        CK(tmp.alloc(&xfb.list, static_cast<size_t>(kExactFallbackRows), "flagged assignment rows"));
-        CK(tmp.alloc(&xfb.nflag, 1, "flagged assignment row count"));
-        CK(tmp.alloc(&xfb.partial, static_cast<size_t>(kExactFallbackRows) * kExactPartialKeys,
-                     "flagged assignment keys"));
-        float* padded = nullptr;
-        if (dim < kDim) CK(tmp.alloc(&padded, static_cast<size_t>(batch) * kDim, "padded rows"));
         for (int64_t start = 0; start < c->n; start += batch) {
             const int nb = static_cast<int>(std::min<int64_t>(batch, c->n - start));
             const float* rows = d_emb + static_cast<size_t>(start) * dim;
@@ -953,34 +1166,36 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
                    "centroid assignment");
         }
         CK_HIP(hipStreamSynchronize(s), "centroid assignment");
-        for (void* p : {static_cast<void*>(cu), static_cast<void*>(nu), static_cast<void*>(nhu), static_cast<void*>(cbu),
-                        static_cast<void*>(ebu), static_cast<void*>(ukey), static_cast<void*>(cnt), static_cast<void*>(flag),
-                        static_cast<void*>(buf), static_cast<void*>(padded), static_cast<void*>(xfb.list),
-                        static_cast<void*>(xfb.nflag), static_cast<void*>(xfb.partial)})
-            if (p) tmp.release(p);
+        tmp.release();
+        tmp.region = region;
+        tmp.region_bytes = region_bytes;
     }
 
     // IVF lists and the cluster-ordered arrays (ivf_pg.cpp:110-126,
     // build_index.cu:328-363)
     {
         uint32_t *keys_out = nullptr, *vals_in = nullptr, *token_doc_u = nullptr;
-        CK(tmp.alloc(&keys_out, n, "sorted assignments"));
-        CK(tmp.alloc(&vals_in, n, "token ids"));
-        CK(dev_alloc(c, c->index_allocs, &c->inv, n, "IVF lists"));
         size_t temp_bytes = 0;
         CK_HIP(launch_sort_assignments(s, labels, c->n, c->n_clusters, keys_out, vals_in, c->inv, nullptr,
                                        &temp_bytes),
                "sort sizing");
         unsigned char* sort_tmp = nullptr;
-        CK(tmp.alloc(&sort_tmp, temp_bytes, "sort scratch"));
+        CK(tmp.carve("sort buffers", [&](Carver& take) {
+            take(keys_out, n);
+            take(vals_in, n);
+            take(token_doc_u, n);
+            take(sort_tmp, temp_bytes);
+        }));
+        CK(dev_carve(c, c->index_allocs, "cluster-order index arrays", [&](Carver& take) {
+            take(c->inv, n);
+            take(c->cluster_pos, K + 1);
+            take(c->codes_clu, n * kCodeBytes);
+            take(c->f1_clu, n);
+            take(c->doc_clu, n);
+        }));
         CK_HIP(launch_sort_assignments(s, labels, c->n, c->n_clusters, keys_out, vals_in, c->inv, sort_tmp,
                                        &temp_bytes),
                "assignment sort");
-        CK(dev_alloc(c, c->index_allocs, &c->cluster_pos, K + 1, "cluster_pos"));
-        CK(dev_alloc(c, c->index_allocs, &c->codes_clu, n * kCodeBytes, "clustered codes"));
-        CK(dev_alloc(c, c->index_allocs, &c->f1_clu, n, "clustered factors"));
-        CK(dev_alloc(c, c->index_allocs, &c->doc_clu, n, "clustered doc ids"));
-        CK(tmp.alloc(&token_doc_u, n, "token documents"));
         CK_HIP(launch_layout(s, keys_out, c->inv, c->n, c->n_clusters, c->doc_ptrs, c->num_docs, c->codes_tok,
                              c->f1_tok, reinterpret_cast<int32_t*>(token_doc_u), c->cluster_pos, c->codes_clu,
                              c->f1_clu, c->doc_clu),
@@ -991,6 +1206,8 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
     CK_HIP(hipStreamSynchronize(s), "index build");
     if (st & 1u) return fail(CHIMERA_ERR_INVALID_ARGUMENT, "Every embedding must be finite and non-zero");
     if (st & 2u) return fail(CHIMERA_ERR_RUNTIME, "Full-code rescale search exceeded its event bound");
+    tmp.release();
+    keep.release();
     return finish_setup(c, *opt, max_batch);
 }
 
@@ -1077,7 +1294,7 @@ int chimera_upload_index(chimera_ctx* c, const chimera_index_desc* d, const chim
                          int32_t max_batch) {
     if (!c || !d || !opt) return fail(CHIMERA_ERR_INVALID_ARGUMENT, "null argument");
     CK(set_device(c));
-    release_index(c);
+    const Rebuild rebuild(c);
     if (d->num_embeddings == 0 || d->num_embeddings > 0x7FFFFFFFull || d->dimension < 64 || d->dimension > 128 ||
         d->num_clusters == 0 || d->num_clusters > d->num_embeddings || d->ex_bits < 1 || d->ex_bits > 7 ||
         d->num_docs == 0) {
@@ -1142,12 +1359,7 @@ int chimera_upload_index(chimera_ctx* c, const chimera_index_desc* d, const chim
            "token-order gather");
     CK_HIP(launch_centroid_norms(c->stream, c->centroids, c->n_clusters, c->norms), "centroid norms");
     CK_HIP(hipStreamSynchronize(c->stream), "index upload");
-    {
-        auto it = std::find(c->index_allocs.begin(), c->index_allocs.end(), static_cast<void*>(tok2pos));
-        c->index_allocs.erase(it);
-        c->bytes -= n * sizeof(uint32_t);
-        (void)hipFree(tok2pos);
-    }
+    dev_free(c, c->index_allocs, tok2pos);
     const int r = finish_setup(c, *opt, max_batch);
     if (r != CHIMERA_OK) {
         // a failed initialisation releases everything (chimera_index.cu:167-172)
@@ -1599,31 +1811,50 @@ int chimera_download_index(chimera_ctx* c, chimera_index_host* h) {
     const size_t n = static_cast<size_t>(c->n);
     const size_t K = static_cast<size_t>(c->n_clusters);
     const size_t width = static_cast<size_t>(1 + c->ex_bits);
-    auto get = [&](void* dst, const void* src, size_t bytes, const char* what) -> int {
-        if (!dst) return CHIMERA_OK;
-        CK_HIP(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost), what);
-        return CHIMERA_OK;
+    std::vector<HostCopy> arrays;
+    auto get = [&](void* dst, const void* src, size_t bytes) {
+        if (dst) arrays.push_back({static_cast<unsigned char*>(dst), static_cast<const unsigned char*>(src), bytes});
     };
-    CK(get(h->cluster_pos, c->cluster_pos, (K + 1) * sizeof(uint64_t), "cluster_pos download"));
-    CK(get(h->one_bit_codes, c->codes_tok, n * kCodeBytes, "one-bit codes download"));
-    CK(get(h->one_bit_factors, c->f1_tok, n * sizeof(float), "one-bit factors download"));
-    CK(get(h->full_codes, c->full_codes, n * 16 * width, "full codes download"));
-    CK(get(h->full_factors, c->full_factors, n * sizeof(float), "full factors download"));
-    CK(get(h->clustered_codes, c->codes_clu, n * kCodeBytes, "clustered codes download"));
-    CK(get(h->clustered_factors, c->f1_clu, n * sizeof(float), "clustered factors download"));
-    CK(get(h->clustered_doc_ids, c->doc_clu, n * sizeof(int32_t), "clustered doc ids download"));
-    CK(get(h->rotated_centroids, c->centroids, K * kDim * sizeof(float), "centroid download"));
-    if (h->inv_list || h->token_to_cluster_pos) {
-        std::vector<uint32_t> local;
-        uint32_t* inv = h->inv_list;
-        if (!inv) {
-            local.resize(n);
-            inv = local.data();
+    get(h->cluster_pos, c->cluster_pos, (K + 1) * sizeof(uint64_t));
+    get(h->one_bit_codes, c->codes_tok, n * kCodeBytes);
+    get(h->one_bit_factors, c->f1_tok, n * sizeof(float));
+    get(h->full_codes, c->full_codes, n * 16 * width);
+    get(h->full_factors, c->full_factors, n * sizeof(float));
+    get(h->clustered_codes, c->codes_clu, n * kCodeBytes);
+    get(h->clustered_factors, c->f1_clu, n * sizeof(float));
+    get(h->clustered_doc_ids, c->doc_clu, n * sizeof(int32_t));
+    get(h->rotated_centroids, c->centroids, K * kDim * sizeof(float));
+    get(h->inv_list, c->inv, n * sizeof(uint32_t));
+    // the token order of the IVF list, made on the device (a scatter of one
+    // pass there, of cache misses here)
+    TempBuffers tmp;
+    tmp.stream = c->stream;
+    uint32_t* pos = nullptr;
+    std::vector<uint32_t> local;
+    const uint32_t* host_inv = nullptr;  // made here when the device has no room for it
+    if (h->token_to_cluster_pos) {
+        if (tmp.alloc(&pos, n, "token positions") == CHIMERA_OK) {
+            CK_HIP(launch_invert(c->stream, c->inv, c->n, pos), "token positions");
+            get(h->token_to_cluster_pos, pos, n * sizeof(uint32_t));
+        } else {
+            if (!h->inv_list) {
+                local.resize(n);
+                get(local.data(), c->inv, n * sizeof(uint32_t));
+            }
+            host_inv = h->inv_list ? h->inv_list : local.data();
         }
-        CK(get(inv, c->inv, n * sizeof(uint32_t), "IVF list download"));
-        if (h->token_to_cluster_pos)
-            for (size_t p = 0; p < n; ++p) h->token_to_cluster_pos[inv[p]] = static_cast<uint32_t>(p);
     }
+    size_t total = 0;
+    for (const HostCopy& a : arrays) total += a.bytes;
+    if (total >= 4 * kSlotBytes && ensure_stage(c, kCopyThreads * kSlotBytes) == CHIMERA_OK) {
+        CK(download_arrays(c, arrays));
+    } else {  // little to copy, or no pinned memory to copy through
+        for (const HostCopy& a : arrays)
+            CK_HIP(hipMemcpyAsync(a.dst, a.src, a.bytes, hipMemcpyDeviceToHost, c->stream), "index download");
+        CK_HIP(hipStreamSynchronize(c->stream), "index download");
+    }
+    if (host_inv)
+        for (size_t p = 0; p < n; ++p) h->token_to_cluster_pos[host_inv[p]] = static_cast<uint32_t>(p);
     return CHIMERA_OK;
 }
 

@@ -202,6 +202,8 @@ hipError_t launch_gather_rows(hipStream_t s, const float* src, int dim, const in
 // scratch size into *temp_bytes.
 hipError_t launch_sort_assignments(hipStream_t s, const uint32_t* labels, int64_t n, int64_t k, uint32_t* keys_out,
                                    uint32_t* vals_in, uint32_t* vals_out, void* temp, size_t* temp_bytes);
+// pos[inv[p]] = p: the position of each token from the token at each position.
+hipError_t launch_invert(hipStream_t s, const uint32_t* inv, int64_t n, uint32_t* pos);
 hipError_t launch_layout(hipStream_t s, const uint32_t* sorted_keys, const uint32_t* inv, int64_t n, int64_t k,
                          const int32_t* doc_ptrs, int64_t m, const uint8_t* codes_tok, const float* f1_tok,
                          int32_t* token_doc, uint64_t* cluster_pos, uint8_t* codes_clu, float* f1_clu,

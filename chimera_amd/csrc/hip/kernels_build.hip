@@ -623,6 +623,11 @@ __global__ void iota_u32_kernel(uint32_t* __restrict__ v, int64_t n) {
     if (i < n) v[i] = static_cast<uint32_t>(i);
 }
 
+__global__ void invert_kernel(const uint32_t* __restrict__ inv, int64_t n, uint32_t* __restrict__ pos) {
+    const int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (p < n) pos[inv[p]] = static_cast<uint32_t>(p);
+}
+
 // cluster_pos[c] = first position of cluster c in the sorted assignments.
 __global__ void cluster_bounds_kernel(const uint32_t* __restrict__ sorted, int64_t n, int64_t k,
                                       uint64_t* __restrict__ cluster_pos) {
@@ -696,6 +701,12 @@ hipError_t launch_sort_assignments(hipStream_t s, const uint32_t* labels, int64_
     if (e != hipSuccess) return e;
     return hipcub::DeviceRadixSort::SortPairs(temp, *temp_bytes, labels, keys_out, vals_in, vals_out,
                                               static_cast<int>(n), 0, end_bit, s);
+}
+
+hipError_t launch_invert(hipStream_t s, const uint32_t* inv, int64_t n, uint32_t* pos) {
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(invert_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, s, inv, n, pos);
+    return hipGetLastError();
 }
 
 hipError_t launch_layout(hipStream_t s, const uint32_t* sorted_keys, const uint32_t* inv, int64_t n, int64_t k,
