@@ -232,7 +232,7 @@ __device__ double rescale_sequential(const RescaleLane& in, const float* sabs, d
     return tbest;
 }
 
-// All events at once. They fall into kBins intervals of [t_start, t_end)
+// All events at once. They fall into kBins (256 or 512) intervals of [t_start, t_end)
 // and one for t >= t_end (each dimension's first event is taken wherever it
 // lies); the sums per interval, and a wave scan over them, give the state
 // (num, den) at the end of every interval. Inside an interval that starts at
@@ -241,8 +241,8 @@ __device__ double rescale_sequential(const RescaleLane& in, const float* sabs, d
 // 0 <= x <= X (X the interval's sum). That curve falls and then rises (the
 // sign of its slope is that of d - tl n + tl x), so max(n^2 / d,
 // (n + X)^2 / (d + 2 tl X)) bounds the interval, and only the intervals
-// whose bound reaches the best interval end are stepped through: 1.1 to 4 of
-// the 257 on Gaussian tokens (ex_bits 1 to 7), with 0 to 17 events.
+// whose bound reaches the best interval end are stepped through: 1.3 to 2.8
+// of the 257 on Gaussian tokens (2.2 of 513 at ex_bits 7).
 //
 // The sums are the sequential ones: the caller has checked that every
 // partial sum of num is a multiple of a power of two below 2^53 of them, so
@@ -259,16 +259,16 @@ __device__ double rescale_sequential(const RescaleLane& in, const float* sabs, d
 // An interval is narrower than 1 / max a = the least spacing of one
 // dimension's events (the range is at most 26 spacings for every ex_bits), so
 // a dimension has at most one event in it.
-constexpr int kBins = 256;
+template <int kBins>
 struct RescaleBins {
     double sum[kBins + 1];    // sum of a_i over the interval's events
     uint32_t cu[kBins + 1];   // events << 16 | sum of u
 };
 
-__device__ double rescale_binned(const RescaleLane& in, RescaleBins& bins, double t_start, double t_end, double num0,
+template <int kBins>
+__device__ double rescale_binned(const RescaleLane& in, RescaleBins<kBins>& bins, double t_start, double t_end, double num0,
                                  double den0, int top, int l) {
     constexpr int kPerLane = kBins / kWave;
-    static_assert(kPerLane == 4, "a lane owns four intervals");
     for (int b = l; b < kBins + 1; b += kWave) {
         bins.sum[b] = 0.0;
         bins.cu[b] = 0u;
@@ -290,36 +290,36 @@ __device__ double rescale_binned(const RescaleLane& in, RescaleBins& bins, doubl
         return b < 0 ? 0 : (b < kBins ? b : kBins - 1);
     };
     wave_lds_sync();
+    // A dimension's events are u = c + 1 .. last: the first wherever it lies,
+    // the others while u <= top and u / a < t_end. The largest u below t_end
+    // is within one of t_end a, so the counts are known before the walk, which
+    // then has one branch a step.
+    auto events_of = [&](float a, double y, int c) {
+        int last = static_cast<int>(t_end * static_cast<double>(a));
+        if (!(time_of(last, a, y) < t_end))
+            --last;
+        else if (time_of(last + 1, a, y) < t_end)
+            ++last;
+        last = last < top ? last : top;
+        return (last > c + 1 ? last : c + 1) - c;
+    };
     {
-        // the lane's events: dimension a's, then dimension b's
-        float a = in.oa;
-        double y = ya;
-        int u = in.ca + 1;
-        double t = time_of(u, a, y);
-        const double tb0 = time_of(in.cb + 1, in.ob, yb);
-        bool second = false, live = true;
-        while (__any(live)) {
-            if (live) {
-                const int b = bin_of(t);
+        const int na = events_of(in.oa, ya, in.ca);
+        const int total = na + events_of(in.ob, yb, in.cb);
+        const int trips = static_cast<int>(wave_all_max(static_cast<float>(total)));
+        for (int i = 0; i < trips; ++i) {
+            const bool second = i >= na;  // dimension a's events, then dimension b's
+            const float a = second ? in.ob : in.oa;
+            const int u = i + (second ? in.cb + 1 - na : in.ca + 1);
+            const int b = bin_of(time_of(u, a, second ? yb : ya));
+            if (i < total) {
                 atomicAdd(&bins.sum[b], static_cast<double>(a));
                 atomicAdd(&bins.cu[b], (1u << 16) + static_cast<uint32_t>(u));
-                // the dimension's next one counts while u <= top and its
-                // time is below t_end
-                ++u;
-                t = time_of(u, a, y);
-                if (!(u <= top && t < t_end)) {
-                    live = !second;
-                    second = true;
-                    a = in.ob;
-                    y = yb;
-                    u = in.cb + 1;
-                    t = tb0;
-                }
             }
         }
     }
     wave_lds_sync();
-    // interval ends: lane l owns intervals 4l .. 4l + 3
+    // interval ends: lane l owns kPerLane consecutive intervals
     double sums[kPerLane];
     uint32_t cu[kPerLane];
     double own = 0.0;
@@ -459,13 +459,14 @@ __device__ double rescale_binned(const RescaleLane& in, RescaleBins& bins, doubl
 //
 // What bounds it is vector-ALU issue of the rescale search (about 2,500
 // instructions a token at ex_bits 4, against 0.6 KB of HBM traffic). Measured
-// on MI355X: 0.88M tokens at ex_bits 4 in 3.6 ms and 2.9M tokens at ex_bits 7
-// in 30.6 ms; one wave per token that took the events one at a time and ran
+// on MI355X: 0.88M tokens at ex_bits 4 in 3.5 ms and 2.9M tokens at ex_bits 7
+// in 25.1 ms; one wave per token that took the events one at a time and ran
 // the three serial sums on one lane took 63.2 and 659 ms. Four waves per SIMD
 // (128 VGPRs) need the 35 KB of LDS that 32 tokens take.
 constexpr int kEncTokens = 32;
 constexpr int kEncWaves = 4;
-__global__ __launch_bounds__(kEncWaves * kWave, 4) void encode_tokens_kernel(
+template <int kBins>
+__global__ __launch_bounds__(kEncWaves * kWave, kBins <= 256 ? 4 : 3) void encode_tokens_kernel(
     const float* __restrict__ emb, int64_t n, int dim, const uint8_t* __restrict__ flips, float fac, int ex_bits,
     uint8_t* __restrict__ codes1, float* __restrict__ f1, uint8_t* __restrict__ full, float* __restrict__ fF,
     uint32_t* __restrict__ status) {
@@ -475,7 +476,7 @@ __global__ __launch_bounds__(kEncWaves * kWave, 4) void encode_tokens_kernel(
     __shared__ float sabs[kEncWaves][kDim];  // the sequential search's copy
     __shared__ float sip[kEncTokens], ssq[kEncTokens];
     __shared__ uint32_t sbad[kEncTokens];
-    __shared__ RescaleBins bins[kEncWaves];
+    __shared__ RescaleBins<kBins> bins[kEncWaves];
     __shared__ uint8_t fl[4 * kDim / 8];
     const int l = lane_id();
     const int w = wave_id();
@@ -674,8 +675,17 @@ hipError_t launch_encode_tokens(hipStream_t s, const float* emb, int64_t n, int 
     const float fac = 1.0F / sqrtf(static_cast<float>(trunc));
     const int64_t want = static_cast<int64_t>(num_cus) * 16;
     const unsigned grid = static_cast<unsigned>(std::min<int64_t>((n + kEncTokens - 1) / kEncTokens, want));
-    hipLaunchKernelGGL(encode_tokens_kernel, dim3(grid), dim3(kEncWaves * kWave), 0, s, emb, n, dim, flips, fac, ex_bits, codes1,
-                       f1, full, fF, status);
+    auto encode = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kEncWaves * kWave), 0, s, emb, n, dim, flips, fac, ex_bits, codes1, f1,
+                           full, fF, status);
+    };
+    // more intervals leave fewer events to step through, which pays from
+    // 7-bit codes on: 2.9M tokens at ex_bits 7 25.1 ms with 512 and 28.9 with
+    // 256, 0.88M at ex_bits 4 3.9 and 3.5 ms
+    if (ex_bits >= 6)
+        encode(encode_tokens_kernel<512>);
+    else
+        encode(encode_tokens_kernel<256>);
     return hipGetLastError();
 }
 
