@@ -91,6 +91,7 @@ struct Workspace {
     uint32_t* sel = nullptr;      // [split] split selection (see CandidateArgs)
     uint64_t* sel_lists = nullptr;  // [split][select_list_cap(k_refine)]
     int split = 0;
+    int cqs = 0;                  // queries of visit counts
     int32_t* rcount = nullptr;    // [B]
     int32_t* rids = nullptr;      // [B * k_refine]
     float* rscore = nullptr;      // [B * k_refine]
@@ -133,13 +134,15 @@ size_t carve_workspace(const WorkspaceShape& sh, unsigned char* base, Workspace*
     Workspace tmp;
     Workspace& x = w ? *w : tmp;
     const size_t B = sh.batch, QS = sh.qs;
+    // the visit counts of a small batch split each query's visits over blocks
+    const size_t CQ = sh.staging ? std::max<size_t>(QS, kCountQueries) : QS;
     if (sh.staging) take(x.queries, B * kQ * sh.dim);
     take(x.rot, B * kQ * kDim);
     take(x.cb1, B * kQ);
     take(x.cbex, B * kQ);
     take(x.lut, B * kLutPerQuery);
     take(x.labels, B * kQ * sh.nprobe);
-    take(x.vcnt, QS * sh.nbk * kQ);
+    take(x.vcnt, CQ * sh.nbk * kQ);
     take(x.vtot, QS);
     take(x.rec, QS * sh.vcap);
     take(x.tcount, QS * sh.nbk);
@@ -152,6 +155,7 @@ size_t carve_workspace(const WorkspaceShape& sh, unsigned char* base, Workspace*
         take(x.sel_lists, sh.split * static_cast<size_t>(select_list_cap(static_cast<int>(sh.k_refine))));
     }
     x.split = static_cast<int>(sh.split);
+    x.cqs = static_cast<int>(CQ);
     take(x.rcount, B);
     take(x.rids, B * sh.k_refine);
     take(x.rscore, B * sh.k_refine);
@@ -642,7 +646,7 @@ CandidateArgs candidate_args(chimera_ctx* c, const Workspace& w) {
     a.rscore = w.rscore;
     a.err = w.err;
     a.num_cus = c->num_cus;
-    a.wqs = w.qs;
+    a.wqs = w.cqs;
     a.sel = w.sel;
     a.sel_lists = w.sel_lists;
     a.sel_queries = w.split;

@@ -131,7 +131,7 @@ struct CandidateArgs {
     float* rscore;
     uint32_t* err;
     int num_cus;
-    int wqs;  // queries the candidate state (vcnt, vtot, rec, ...) holds
+    int wqs;  // queries of visit counts that vcnt holds
     uint32_t* sel;        // [sel_queries][kSelectWords] split selection: S histogram, list count (null: not held)
     uint64_t* sel_lists;  // [sel_queries][select_list_cap(k_refine)]
     int sel_queries;
@@ -142,6 +142,7 @@ struct CandidateArgs {
 constexpr int kSelectBins = 4096;
 constexpr int kSelectWords = kSelectBins + 32;
 constexpr int kSelectSplitQueries = 1024;
+constexpr int kCountQueries = 256;  // visit counts are held for at least so many queries
 constexpr int64_t kSelectSplitDocs = 8'000'000;
 int cand_buckets(int64_t num_docs, int blog);
 // Bucket size (log2) of the candidate stage for an index: the largest in
