@@ -79,7 +79,7 @@ PROBE_WORKLOADS = {
 
 # kernel behind each single-kernel stage (names as rocprofv3 reports them)
 STAGE_KERNELS = {
-    "probe_scan": "chimera::probe_mfma_kernel<1, 4>",
+    "probe_scan": "chimera::probe_mfma_kernel<1, 4, 1>",
     "count": "chimera::cand_count_kernel",
     "emit": "chimera::cand_emit_staged_kernel",
     "reduce": "chimera::cand_reduce_kernel<8>",
