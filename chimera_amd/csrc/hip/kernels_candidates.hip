@@ -1562,7 +1562,7 @@ hipError_t configure_candidate_kernels(int nbk, int k_refine) {
 // Visit ranges per (query, token) in the count and emit kernels of a
 // sub-batch of qs queries: doubled, up to kMaxParts, while their grids stay
 // within two blocks per CU and the visit counts of qs x parts queries fit
-// the candidate state (which holds wqs queries). One query at docs2m takes
+// the visit counts held (wqs queries). One query at docs2m takes
 // 16 parts: 512 blocks instead of 32 on one XCD.
 constexpr int kMaxParts = 16;
 int cand_parts(int qs, int num_cus, int wqs) {
