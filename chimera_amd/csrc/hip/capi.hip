@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -271,30 +272,42 @@ void free_list(std::vector<DevBlock>& list) {
     list.clear();
 }
 
+// Device memory for the context; the spares of a build or upload give way to
+// it.
+int device_malloc(chimera_ctx* c, void** p, size_t bytes, const char* what) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && !c->spare.empty()) {
+        (void)hipGetLastError();
+        free_list(c->spare);
+        e = hipMalloc(p, bytes);
+    }
+    if (e == hipSuccess) return CHIMERA_OK;
+    return fail(CHIMERA_ERR_HIP, std::string("hipMalloc of ") + what + " (" + std::to_string(bytes) +
+                                     " bytes) failed: " + hipGetErrorString(e));
+}
+
+// Bytes of a spare block that may stay unused (at most a quarter): what an
+// allocation is rounded up to, so that an index built over spares takes no
+// more memory than a first one.
+constexpr size_t kSpareWaste = size_t{2} << 20;
+
 template <typename T>
-int dev_alloc(chimera_ctx* c, std::vector<DevBlock>& list, T** p, size_t count, const char* what) {
+int dev_alloc(chimera_ctx* c, std::vector<DevBlock>& list, T** p, size_t count, const char* what,
+              size_t most_waste = kSpareWaste) {
     *p = nullptr;
     if (count == 0) count = 1;
     const size_t bytes = count * sizeof(T);
     DevBlock block{nullptr, bytes};
-    // the smallest spare block that holds it without wasting a quarter
+    // the smallest spare block that holds it without wasting more
+    const size_t waste = std::min(bytes / 4, most_waste);
     auto fit = c->spare.end();
     for (auto it = c->spare.begin(); it != c->spare.end(); ++it)
-        if (it->bytes >= bytes && it->bytes - bytes <= bytes / 4 && (fit == c->spare.end() || it->bytes < fit->bytes)) fit = it;
+        if (it->bytes >= bytes && it->bytes - bytes <= waste && (fit == c->spare.end() || it->bytes < fit->bytes)) fit = it;
     if (fit != c->spare.end()) {
         block = *fit;
         c->spare.erase(fit);
     } else {
-        hipError_t e = hipMalloc(&block.ptr, bytes);
-        if (e != hipSuccess && !c->spare.empty()) {
-            (void)hipGetLastError();
-            free_list(c->spare);
-            e = hipMalloc(&block.ptr, bytes);
-        }
-        if (e != hipSuccess) {
-            return fail(CHIMERA_ERR_HIP, std::string("hipMalloc of ") + what + " (" + std::to_string(bytes) +
-                                             " bytes) failed: " + hipGetErrorString(e));
-        }
+        CK(device_malloc(c, &block.ptr, bytes, what));
     }
     list.push_back(block);
     c->bytes += block.bytes;
@@ -448,27 +461,20 @@ int collect_stage_times(chimera_ctx* c) {
 
 // Device buffers that live for one call; freed after the stream drains.
 struct TempBuffers {
-    hipStream_t stream = nullptr;
+    chimera_ctx* ctx;
     std::vector<void*> ptrs;
     // memory of the context that nothing else uses meanwhile: carve() takes
     // from it what fits
     unsigned char* region = nullptr;
     size_t region_bytes = 0;
-    ~TempBuffers() {
-        if (stream) (void)hipStreamSynchronize(stream);
-        for (void* p : ptrs) (void)hipFree(p);
-    }
+    explicit TempBuffers(chimera_ctx* c) : ctx(c) {}
+    ~TempBuffers() { release(); }
     template <typename T>
     int alloc(T** p, size_t count, const char* what) {
         *p = nullptr;
         if (count == 0) count = 1;
         void* ptr = nullptr;
-        const hipError_t e = hipMalloc(&ptr, count * sizeof(T));
-        if (e != hipSuccess) {
-            return fail(CHIMERA_ERR_HIP, std::string("hipMalloc of ") + what + " (" +
-                                             std::to_string(count * sizeof(T)) + " bytes) failed: " +
-                                             hipGetErrorString(e));
-        }
+        CK(device_malloc(ctx, &ptr, count * sizeof(T), what));
         ptrs.push_back(ptr);
         *p = static_cast<T*>(ptr);
         return CHIMERA_OK;
@@ -490,7 +496,7 @@ struct TempBuffers {
         return CHIMERA_OK;
     }
     void release() {
-        if (stream) (void)hipStreamSynchronize(stream);
+        (void)hipStreamSynchronize(ctx->stream);
         for (void* p : ptrs) (void)hipFree(p);
         ptrs.clear();
     }
@@ -983,7 +989,10 @@ int finish_setup(chimera_ctx* c, const chimera_search_options& o, int32_t max_ba
                             static_cast<size_t>(opt->k_refine), static_cast<size_t>(c->fb_cap), true,
                             static_cast<size_t>(std::min(c->qs, kSelectSplitQueries)), c->blog};
     unsigned char* block = nullptr;
-    CK(dev_alloc(c, c->ws_allocs, &block, carve_workspace(sh, nullptr, nullptr), "search workspace"));
+    // its size varies with the cluster sizes from build to build; it comes
+    // last, so a quarter left over takes no room from anything
+    const size_t ws_bytes = carve_workspace(sh, nullptr, nullptr);
+    CK(dev_alloc(c, c->ws_allocs, &block, ws_bytes, "search workspace", SIZE_MAX));
     carve_workspace(sh, block, &c->ws);
     CK_HIP(launch_fill_u32(c->stream, reinterpret_cast<uint32_t*>(c->ws.rcount), max_batch, 0u), "clearing refined counts");
     CK_HIP(launch_fill_u32(c->stream, c->ws.err, 1, 0u), "clearing status");
@@ -1062,9 +1071,7 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
     // the build's own buffers: labels through the whole build, then those of
     // the assignment and those of the sort, in the probe's record area where
     // they fit (no search runs meanwhile)
-    TempBuffers keep, tmp;
-    keep.stream = s;
-    tmp.stream = s;
+    TempBuffers keep(c), tmp(c);
     {
         const ProbePlan plan = plan_probe_mfma(max_batch * kQ, c->n_clusters, opt->nprobe, c->num_cus);
         if (plan.usable) {
@@ -1501,8 +1508,7 @@ int chimera_search_trace(chimera_ctx* c, const float* queries, int32_t nq, int32
     std::vector<int32_t> counts(static_cast<size_t>(c->qs));
     // dense candidate lists of a sub-batch, compacted on the device
     const int64_t tcap = std::max<int64_t>(1, std::min<int64_t>(tr->cand_capacity, c->num_docs));
-    TempBuffers tmp;
-    tmp.stream = s;
+    TempBuffers tmp(c);
     int32_t* d_cand = nullptr;
     float* d_score = nullptr;
     if (tr->candidates || tr->candidate_scores) {
@@ -1831,8 +1837,7 @@ int chimera_download_index(chimera_ctx* c, chimera_index_host* h) {
     get(h->inv_list, c->inv, n * sizeof(uint32_t));
     // the token order of the IVF list, made on the device (a scatter of one
     // pass there, of cache misses here)
-    TempBuffers tmp;
-    tmp.stream = c->stream;
+    TempBuffers tmp(c);
     uint32_t* pos = nullptr;
     std::vector<uint32_t> local;
     const uint32_t* host_inv = nullptr;  // made here when the device has no room for it
