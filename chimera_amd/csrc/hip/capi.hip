@@ -126,6 +126,12 @@ struct Carver {
         off += std::max<size_t>(count, 1) * sizeof(T);
     }
     size_t bytes() const { return (off + 255) / 256 * 256; }
+    template <typename Lay>
+    static size_t size(Lay&& lay) {
+        Carver sizes;
+        lay(sizes);
+        return sizes.bytes();
+    }
 };
 
 // Bytes of a workspace of this shape; with a base, also the pointers into it.
@@ -329,10 +335,8 @@ void dev_free(chimera_ctx* c, std::vector<DevBlock>& list, void* ptr) {
 // One allocation of the context's `list` for the arrays that `lay` takes.
 template <typename Lay>
 int dev_carve(chimera_ctx* c, std::vector<DevBlock>& list, const char* what, Lay&& lay) {
-    Carver sizes;
-    lay(sizes);
     Carver arrays;
-    CK(dev_alloc(c, list, &arrays.base, sizes.bytes(), what));
+    CK(dev_alloc(c, list, &arrays.base, Carver::size(lay), what));
     lay(arrays);
     return CHIMERA_OK;
 }
@@ -482,15 +486,14 @@ struct TempBuffers {
     // one allocation for the arrays that `lay` takes
     template <typename Lay>
     int carve(const char* what, Lay&& lay) {
-        Carver sizes;
-        lay(sizes);
+        const size_t bytes = Carver::size(lay);
         Carver arrays;
-        if (sizes.bytes() <= region_bytes) {
+        if (bytes <= region_bytes) {
             arrays.base = region;
-            region += sizes.bytes();
-            region_bytes -= sizes.bytes();
+            region += bytes;
+            region_bytes -= bytes;
         } else {
-            CK(alloc(&arrays.base, sizes.bytes(), what));
+            CK(alloc(&arrays.base, bytes, what));
         }
         lay(arrays);
         return CHIMERA_OK;
@@ -1069,15 +1072,61 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
     const size_t width = static_cast<size_t>(1 + ex_bits);
     hipStream_t s = c->stream;
     // the build's own buffers: labels through the whole build, then those of
-    // the assignment and those of the sort, in the probe's record area where
-    // they fit (no search runs meanwhile)
+    // the assignment and those of the sort
+    uint32_t *status = nullptr, *labels = nullptr;
+    int64_t* d_ids = nullptr;
+    auto lay_labels = [&](Carver& take) {
+        take(status, 1);
+        take(labels, n);
+        take(d_ids, K);
+    };
+    const int64_t batch = std::min<int64_t>(c->n, kAssignBatch);
+    const ProbePlan full_plan = plan_assign_top1(static_cast<int>(batch), c->n_clusters, c->num_cus);
+    const size_t sub_rows = probe_sublist_rows(static_cast<int>(batch), c->num_cus);
+    float *cu = nullptr, *nu = nullptr, *nhu = nullptr, *padded = nullptr;
+    uint16_t* cbu = nullptr;
+    uint32_t *ebu = nullptr, *ukey = nullptr, *cnt = nullptr, *flag = nullptr;
+    uint2* buf = nullptr;
+    ExactFallback xfb;
+    xfb.list_cap = kExactFallbackRows;
+    auto lay_assign = [&](Carver& take) {
+        take(cu, K * kDim);
+        take(nu, K);
+        take(nhu, K);
+        take(cbu, K * kDim);
+        take(ebu, 1);
+        take(ukey, static_cast<size_t>(batch));
+        take(cnt, sub_rows * 2);
+        take(flag, static_cast<size_t>(batch));
+        take(buf, sub_rows * 2 * static_cast<size_t>(full_plan.lane_cap));
+        take(xfb.list, static_cast<size_t>(kExactFallbackRows));
+        take(xfb.nflag, 1);
+        take(xfb.partial, static_cast<size_t>(kExactFallbackRows) * kExactPartialKeys);
+        if (dim < kDim) take(padded, static_cast<size_t>(batch) * kDim);
+    };
+    uint32_t *keys_out = nullptr, *vals_in = nullptr, *token_doc_u = nullptr;
+    unsigned char* sort_tmp = nullptr;
+    size_t sort_bytes = 0;
+    CK_HIP(launch_sort_assignments(s, labels, c->n, c->n_clusters, keys_out, vals_in, c->inv, nullptr, &sort_bytes),
+           "sort sizing");
+    auto lay_sort = [&](Carver& take) {
+        take(keys_out, n);
+        take(vals_in, n);
+        take(token_doc_u, n);
+        take(sort_tmp, sort_bytes);
+    };
+    // Where all of it fits the probe's record area it lives there (no search
+    // runs meanwhile). Else the probe's buffers come after it: held beside
+    // it they would only raise the build's peak of memory.
     TempBuffers keep(c), tmp(c);
     {
         const ProbePlan plan = plan_probe_mfma(max_batch * kQ, c->n_clusters, opt->nprobe, c->num_cus);
-        if (plan.usable) {
+        const size_t record_bytes =
+            plan.usable ? probe_sublist_rows(max_batch * kQ, c->num_cus) * 2 * static_cast<size_t>(plan.lane_cap) * 32 : 0;
+        if (Carver::size(lay_labels) + std::max(Carver::size(lay_assign), Carver::size(lay_sort)) <= record_bytes) {
             CK(alloc_probe(c, plan, max_batch));
             keep.region = reinterpret_cast<unsigned char*>(c->p_rval);
-            keep.region_bytes = probe_sublist_rows(max_batch * kQ, c->num_cus) * 2 * static_cast<size_t>(plan.lane_cap) * 32;
+            keep.region_bytes = record_bytes;
         }
     }
 
@@ -1097,13 +1146,7 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
     CK_HIP(hipMemsetAsync(c->f1_tok + n, 0, kRefinePadTokens * sizeof(float), s), "factor padding");
     CK_HIP(hipMemsetAsync(c->full_codes + n * 16 * width, 0, kFullbitPadTokens * 16 * width, s), "full code padding");
     CK_HIP(hipMemsetAsync(c->full_factors + n, 0, kFullbitPadTokens * sizeof(float), s), "full factor padding");
-    uint32_t *status = nullptr, *labels = nullptr;
-    int64_t* d_ids = nullptr;
-    CK(keep.carve("build labels", [&](Carver& take) {
-        take(status, 1);
-        take(labels, n);
-        take(d_ids, K);
-    }));
+    CK(keep.carve("build labels", lay_labels));
     unsigned char* const region = keep.region;
     const size_t region_bytes = keep.region_bytes;
     tmp.region = region;
@@ -1122,34 +1165,7 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
 
     // nearest-centroid assignment in the input space (build_index.cu:186-219)
     {
-        float* cu = nullptr;
-        float* nu = nullptr;
-        float* nhu = nullptr;
-        uint16_t* cbu = nullptr;
-        uint32_t* ebu = nullptr;
-        const int64_t batch = std::min<int64_t>(c->n, kAssignBatch);
-        const ProbePlan full_plan = plan_assign_top1(static_cast<int>(batch), c->n_clusters, c->num_cus);
-        const size_t sub_rows = probe_sublist_rows(static_cast<int>(batch), c->num_cus);
-        uint32_t *ukey = nullptr, *cnt = nullptr, *flag = nullptr;
-        uint2* buf = nullptr;
-        float* padded = nullptr;
-        ExactFallback xfb;
-        xfb.list_cap = kExactFallbackRows;
-        CK(tmp.carve("assignment buffers", [&](Carver& take) {
-            take(cu, K * kDim);
-            take(nu, K);
-            take(nhu, K);
-            take(cbu, K * kDim);
-            take(ebu, 1);
-            take(ukey, static_cast<size_t>(batch));
-            take(cnt, sub_rows * 2);
-            take(flag, static_cast<size_t>(batch));
-            take(buf, sub_rows * 2 * static_cast<size_t>(full_plan.lane_cap));
-            take(xfb.list, static_cast<size_t>(kExactFallbackRows));
-            take(xfb.nflag, 1);
-            take(xfb.partial, static_cast<size_t>(kExactFallbackRows) * kExactPartialKeys);
-            if (dim < kDim) take(padded, static_cast<size_t>(batch) * kDim);
-        }));
+        CK(tmp.carve("assignment buffers", lay_assign));
         CK_HIP(launch_gather_rows(s, d_emb, dim, d_ids, c->n_clusters, nullptr, false, cu), "centroid gather");
         CK_HIP(launch_centroid_norms(s, cu, c->n_clusters, nu), "centroid norms");
         CK_HIP(launch_probe_centroids(s, cu, nu, c->n_clusters, cbu, nhu, ebu), "bf16 centroids");
@@ -1185,18 +1201,7 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
     // IVF lists and the cluster-ordered arrays (ivf_pg.cpp:110-126,
     // build_index.cu:328-363)
     {
-        uint32_t *keys_out = nullptr, *vals_in = nullptr, *token_doc_u = nullptr;
-        size_t temp_bytes = 0;
-        CK_HIP(launch_sort_assignments(s, labels, c->n, c->n_clusters, keys_out, vals_in, c->inv, nullptr,
-                                       &temp_bytes),
-               "sort sizing");
-        unsigned char* sort_tmp = nullptr;
-        CK(tmp.carve("sort buffers", [&](Carver& take) {
-            take(keys_out, n);
-            take(vals_in, n);
-            take(token_doc_u, n);
-            take(sort_tmp, temp_bytes);
-        }));
+        CK(tmp.carve("sort buffers", lay_sort));
         CK(dev_carve(c, c->index_allocs, "cluster-order index arrays", [&](Carver& take) {
             take(c->inv, n);
             take(c->cluster_pos, K + 1);
@@ -1205,7 +1210,7 @@ int build_on_device(chimera_ctx* c, const float* d_emb, uint64_t n_, uint64_t di
             take(c->doc_clu, n);
         }));
         CK_HIP(launch_sort_assignments(s, labels, c->n, c->n_clusters, keys_out, vals_in, c->inv, sort_tmp,
-                                       &temp_bytes),
+                                       &sort_bytes),
                "assignment sort");
         CK_HIP(launch_layout(s, keys_out, c->inv, c->n, c->n_clusters, c->doc_ptrs, c->num_docs, c->codes_tok,
                              c->f1_tok, reinterpret_cast<int32_t*>(token_doc_u), c->cluster_pos, c->codes_clu,

@@ -83,3 +83,21 @@ build(ctx, 200_000)
 assert hip.host_hip_used() <= need
 assert ctx.search(zeros(8), 10)[0].shape == (8, 10)
 """)
+
+
+def test_the_probe_buffers_do_not_add_to_a_builds_scratch(host_hip):
+    """Where the scratch does not fit the probe's record area, the probe's
+    buffers (larger for larger batches) come after it."""
+    host_hip("""
+hip.host_hip_set_cus(4)
+capacity(1 << 40)
+peaks = []
+for batch in (8, 512):
+    ctx = context(max_batch=batch)
+    hip.host_hip_reset_peak()
+    build(ctx, 200_000)
+    peaks.append(hip.host_hip_peak())
+    assert hip.host_hip_used() < peaks[-1]  # the build is the peak, not what it leaves
+    ctx.close()
+assert abs(peaks[1] - peaks[0]) < 1 << 20, peaks
+""")
