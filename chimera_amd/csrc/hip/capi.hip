@@ -979,6 +979,9 @@ int finish_setup(chimera_ctx* c, const chimera_search_options& o, int32_t max_ba
     // one sub-batch
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = size_t{8} << 30;
+    // (the spares left are free to take: what the context held before does
+    // not size this index's sub-batches)
+    for (const DevBlock& b : c->spare) free_b += b.bytes;
     const int64_t budget = std::max<int64_t>(int64_t{1} << 30, std::min<int64_t>(int64_t{64} << 30,
                                                                                  static_cast<int64_t>(free_b / 2)));
     int qs = static_cast<int>(std::max<int64_t>(8, std::min<int64_t>(budget / std::max<int64_t>(per_query, 1), 4096)));

@@ -87,6 +87,13 @@ std::function<void()> run(const std::string& name, void** args) {
             for (int64_t p = 0; p < n; ++p) pos[inv[p]] = static_cast<uint32_t>(p);
         };
     }
+    if (name.find("cluster_bounds_kernel") != std::string::npos) {  // (sorted, n, k, cluster_pos): clusters of one size
+        const int64_t n = *static_cast<int64_t*>(args[1]), k = *static_cast<int64_t*>(args[2]);
+        auto* pos = *static_cast<uint64_t**>(args[3]);
+        return [=] {
+            for (int64_t c = 0; c <= k; ++c) pos[c] = static_cast<uint64_t>(n * c / k);
+        };
+    }
     return [] {};
 }
 

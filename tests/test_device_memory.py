@@ -92,12 +92,45 @@ def test_the_probe_buffers_do_not_add_to_a_builds_scratch(host_hip):
 hip.host_hip_set_cus(4)
 capacity(1 << 40)
 peaks = []
-for batch in (8, 512):
+for batch in (8, 256):
     ctx = context(max_batch=batch)
     hip.host_hip_reset_peak()
-    build(ctx, 200_000)
+    build(ctx, 200_000, clusters=50_000)
     peaks.append(hip.host_hip_peak())
     assert hip.host_hip_used() < peaks[-1]  # the build is the peak, not what it leaves
     ctx.close()
 assert abs(peaks[1] - peaks[0]) < 1 << 20, peaks
+""")
+
+
+def test_a_rebuild_plans_the_sub_batches_of_a_first_build(host_hip):
+    """The queries per sub-batch come from the free memory, of which the
+    blocks of the replaced index are part."""
+    host_hip("""
+capacity(20 << 30)
+large, small = dict(docs=2_000_000, doc_len=3), dict(docs=20_000)
+
+def plan(ctx):
+    hip.host_hip_reset_launches()
+    ctx.search(zeros(2048), 10)
+    return hip.host_hip_launches(b"cand_count"), ctx.memory_usage()
+
+fresh = context(max_batch=2048)
+build(fresh, **large)
+want = plan(fresh)
+assert want[0] == 2  # the memory bounds them
+fresh.close()
+ctx = context(max_batch=2048)
+build(ctx, **large)
+build(ctx, **small)
+build(ctx, **large)
+assert plan(ctx) == want
+build(ctx, **large)
+assert plan(ctx) == want
+build(ctx, docs=3_000_000, doc_len=2)
+other = plan(ctx)
+ctx.close()
+fresh = context(max_batch=2048)
+build(fresh, docs=3_000_000, doc_len=2)
+assert plan(fresh)[0] == other[0]
 """)
