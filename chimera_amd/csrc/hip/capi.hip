@@ -279,7 +279,9 @@ void free_list(std::vector<DevBlock>& list) {
 }
 
 // Device memory for the context; the spares of a build or upload give way to
-// it.
+// it. A failure is reported here and leaves no HIP error behind: a caller may
+// go on without the memory, and the check after its next launch would report
+// it again.
 int device_malloc(chimera_ctx* c, void** p, size_t bytes, const char* what) {
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess && !c->spare.empty()) {
@@ -288,6 +290,7 @@ int device_malloc(chimera_ctx* c, void** p, size_t bytes, const char* what) {
         e = hipMalloc(p, bytes);
     }
     if (e == hipSuccess) return CHIMERA_OK;
+    (void)hipGetLastError();
     return fail(CHIMERA_ERR_HIP, std::string("hipMalloc of ") + what + " (" + std::to_string(bytes) +
                                      " bytes) failed: " + hipGetErrorString(e));
 }
@@ -774,11 +777,17 @@ int ensure_stage(chimera_ctx* c, size_t host) {
     c->h_stage_bytes = 0;
     const size_t bytes = (host + 4095) / 4096 * 4096;
     void* p = nullptr;
-    CK_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault), "pinned staging buffer");
+    // (the callers go on where either fails, so neither error stays set)
+    const hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocDefault);
+    if (e != hipSuccess) (void)hipGetLastError();
+    CK_HIP(e, "pinned staging buffer");
     c->h_stage = static_cast<unsigned char*>(p);
     c->h_stage_bytes = bytes;
     void* dp = nullptr;
-    c->d_stage = hipHostGetDevicePointer(&dp, p, 0) == hipSuccess ? static_cast<unsigned char*>(dp) : nullptr;
+    if (hipHostGetDevicePointer(&dp, p, 0) == hipSuccess)
+        c->d_stage = static_cast<unsigned char*>(dp);
+    else
+        (void)hipGetLastError();
     return CHIMERA_OK;
 }
 
@@ -1629,8 +1638,7 @@ int chimera_device_alloc(chimera_ctx* c, void** ptr, size_t bytes) {
     if (!c || !ptr) return fail(CHIMERA_ERR_INVALID_ARGUMENT, "null argument");
     CK(set_device(c));
     *ptr = nullptr;
-    CK_HIP(hipMalloc(ptr, bytes ? bytes : 1), "hipMalloc");
-    return CHIMERA_OK;
+    return device_malloc(c, ptr, bytes ? bytes : 1, "a caller's buffer");
 }
 
 int chimera_device_free(chimera_ctx* c, void* ptr) {

@@ -134,3 +134,52 @@ fresh = context(max_batch=2048)
 build(fresh, docs=3_000_000, doc_len=2)
 assert plan(fresh)[0] == other[0]
 """)
+
+
+@pytest.mark.parametrize("refuse", ["host_hip_refuse_malloc(C.c_size_t(4 * ctx.n), C.c_size_t(4 * ctx.n))",
+                                    "host_hip_refuse_host(1)"])
+def test_a_download_that_falls_back_leaves_no_error(host_hip, refuse):
+    """Without room for the token positions, or without pinned memory, the
+    download takes another way; the error it met is not the next call's."""
+    host_hip(f"""
+ctx = context()
+build(ctx, 20_000)
+want = ctx.download()
+ctx.close()
+ctx = context()
+build(ctx, 20_000)
+hip.{refuse}
+got = ctx.download()
+assert all(np.array_equal(got[k], want[k]) for k in want)
+assert ctx.search(zeros(8), 10)[0].shape == (8, 10)
+""")
+
+
+def test_a_search_without_a_device_view_of_its_staging_buffer(host_hip):
+    host_hip("""
+ctx = context()
+build(ctx, 20_000)
+hip.host_hip_refuse_pointer(1)
+assert ctx.search(zeros(2), 10)[0].shape == (2, 10)
+assert ctx.search(zeros(2), 10)[0].shape == (2, 10)
+""")
+
+
+def test_a_failed_build_leaves_no_error_to_other_contexts(host_hip):
+    host_hip("""
+ctx, other = context(), context()
+build(ctx, 20_000)
+capacity(hip.host_hip_used() + (64 << 20))
+try:
+    build(other, 200_000)
+    raise AssertionError("no room for it")
+except capi.ChimeraError as e:
+    assert e.code == capi.ERR_HIP and "out of memory" in str(e)
+assert ctx.search(zeros(8), 10)[0].shape == (8, 10)
+try:
+    ctx.alloc(1 << 40)
+    raise AssertionError("no room for it")
+except capi.ChimeraError as e:
+    assert e.code == capi.ERR_HIP and "out of memory" in str(e)
+assert ctx.search(zeros(8), 10)[0].shape == (8, 10)
+""")
