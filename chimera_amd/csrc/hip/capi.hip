@@ -865,8 +865,10 @@ int download_arrays(chimera_ctx* c, const std::vector<HostCopy>& arrays) {
     for (std::thread& t : threads) t.join();
     for (hipEvent_t ev : landed)
         if (ev) (void)hipEventDestroy(ev);
+    // (on the stream, whose earlier work may still be making an array)
     for (; done < n && e == hipSuccess; ++done)
-        e = hipMemcpy(chunks[done].dst, chunks[done].src, chunks[done].bytes, hipMemcpyDeviceToHost);
+        e = hipMemcpyAsync(chunks[done].dst, chunks[done].src, chunks[done].bytes, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e == hipSuccess) e = static_cast<hipError_t>(error.load());
     CK_HIP(e, "index download");
     return CHIMERA_OK;

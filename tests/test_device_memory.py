@@ -183,3 +183,26 @@ except capi.ChimeraError as e:
     assert e.code == capi.ERR_HIP and "out of memory" in str(e)
 assert ctx.search(zeros(8), 10)[0].shape == (8, 10)
 """)
+
+
+@pytest.mark.parametrize("threads", [0, 3])
+def test_a_download_with_too_few_threads_keeps_the_order(host_hip, threads):
+    """Without threads for every slot of the ring the rest is copied by the
+    caller, after the kernel that makes the token positions."""
+    host_hip(f"""
+import resource
+ctx = context()
+build(ctx, 20_000)
+want = ctx.download()
+assert want["token_to_cluster_pos"].any()
+stack, libc = 4 << 30, C.CDLL(None)
+attr = (C.c_char * 64)()
+assert libc.pthread_attr_init(attr) == 0
+assert libc.pthread_attr_setstacksize(attr, C.c_size_t(stack)) == 0
+assert libc.pthread_setattr_default_np(attr) == 0  # later threads' stacks
+size = int(open("/proc/self/statm").read().split()[0]) * 4096
+limit = size + {threads} * (stack + (1 << 20)) + (1 << 30)
+resource.setrlimit(resource.RLIMIT_AS, (limit, limit))  # room for so many of them
+got = ctx.download()
+assert all(np.array_equal(got[k], want[k]) for k in want)
+""")
