@@ -1022,7 +1022,7 @@ int finish_setup(chimera_ctx* c, const chimera_search_options& o, int32_t max_ba
 
 
 // Rows per assignment launch: one row block for every CU twice over on 256
-// CUs, so that the candidate buffer (2 KB a row) stays at 0.5 GB.
+// CUs, so that the candidate buffer (4 KB a row) stays at 1.1 GB.
 constexpr int64_t kAssignBatch = int64_t{1} << 18;
 
 // Index build on the device (build_index.cu:394-501 with the CAGRA

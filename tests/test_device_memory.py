@@ -206,3 +206,13 @@ resource.setrlimit(resource.RLIMIT_AS, (limit, limit))  # room for so many of th
 got = ctx.download()
 assert all(np.array_equal(got[k], want[k]) for k in want)
 """)
+
+
+def test_assignment_lists_hold_256_candidates(host_hip):
+    """Repeated tokens put many centroids within a row's margin; up to 256 of
+    them in one of its lists keep the row off the exact recomputation."""
+    host_hip("""
+ctx = context()
+build(ctx, 20_000)
+assert hip.host_hip_lane_cap() == 256
+""")

@@ -32,3 +32,26 @@ def test_labels_equal_the_host_build(chimera_mod, n, k, dim, spread):
     ctx.close()
     assert np.array_equal(got["cluster_pos"], ref["cluster_pos"])
     assert np.array_equal(got["inv_list"], ref["inv_list"])
+
+
+# rows of 258 row blocks take one centroid split, so two lists hold a row's
+# candidates: half of the repeats each, on either side of 128 and of the 256
+# that a list holds (past it, the rows are recomputed exactly)
+@pytest.mark.parametrize("repeats", [250, 262, 506, 520])
+def test_many_equal_centroids(chimera_mod, repeats):
+    n, k, dim = 132_000, 700, 128
+    rng = np.random.default_rng(repeats)
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    ids = np.asarray(chimera_mod._sample_centroid_ids(n, k), np.int64)
+    near = rng.permutation(n)[: n // 2]
+    x[near] = x[0] + np.float32(1e-2) * rng.standard_normal((near.size, dim)).astype(np.float32)
+    x[ids[rng.permutation(k)[:repeats]]] = x[0]
+    lens = np.full(n // 20, 20, np.int32)
+    print(f"{repeats} equal centroids of {k}", flush=True)
+    ref = chimera_mod._build_index(x, lens.tolist(), k, 1)
+    ctx = capi.Context(None, 1, 4, 2, 1, max_batch=1)
+    ctx.build(x, lens, k, 1)
+    got = ctx.download(fields=("cluster_pos", "inv_list"))
+    ctx.close()
+    assert np.array_equal(got["cluster_pos"], ref["cluster_pos"])
+    assert np.array_equal(got["inv_list"], ref["inv_list"])
