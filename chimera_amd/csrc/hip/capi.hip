@@ -108,6 +108,7 @@ struct Workspace {
 struct WorkspaceShape {
     size_t batch, qs, dim, nprobe, nbk, vcap, k_refine, fb_cap;
     bool staging;  // query staging and result counts of the host entry points
+    size_t counts;  // queries of visit counts
     size_t split;  // queries of the split selection's state (0: none)
     int blog;      // documents per candidate bucket = 2^blog
 };
@@ -141,15 +142,13 @@ size_t carve_workspace(const WorkspaceShape& sh, unsigned char* base, Workspace*
     Workspace tmp;
     Workspace& x = w ? *w : tmp;
     const size_t B = sh.batch, QS = sh.qs;
-    // the visit counts of a small batch split each query's visits over blocks
-    const size_t CQ = sh.staging ? std::max<size_t>(QS, kCountQueries) : QS;
     if (sh.staging) take(x.queries, B * kQ * sh.dim);
     take(x.rot, B * kQ * kDim);
     take(x.cb1, B * kQ);
     take(x.cbex, B * kQ);
     take(x.lut, B * kLutPerQuery);
     take(x.labels, B * kQ * sh.nprobe);
-    take(x.vcnt, CQ * sh.nbk * kQ);
+    take(x.vcnt, sh.counts * sh.nbk * kQ);
     take(x.vtot, QS);
     take(x.rec, QS * sh.vcap);
     take(x.tcount, QS * sh.nbk);
@@ -162,7 +161,7 @@ size_t carve_workspace(const WorkspaceShape& sh, unsigned char* base, Workspace*
         take(x.sel_lists, sh.split * static_cast<size_t>(select_list_cap(static_cast<int>(sh.k_refine))));
     }
     x.split = static_cast<int>(sh.split);
-    x.cqs = static_cast<int>(CQ);
+    x.cqs = static_cast<int>(sh.counts);
     take(x.rcount, B);
     take(x.rids, B * sh.k_refine);
     take(x.rscore, B * sh.k_refine);
@@ -993,18 +992,25 @@ int finish_setup(chimera_ctx* c, const chimera_search_options& o, int32_t max_ba
     // (the spares left are free to take: what the context held before does
     // not size this index's sub-batches)
     for (const DevBlock& b : c->spare) free_b += b.bytes;
+    // (less what is held beside it: the split selection's state and the visit
+    // counts past the sub-batch's)
+    const int maxb8 = (max_batch + 7) / 8 * 8;
+    const int split = std::min(maxb8, select_split_queries(c->num_docs));
+    const int64_t beside = static_cast<int64_t>(split) * (kSelectWords * 4 + int64_t{8} * select_list_cap(opt->k_refine)) +
+                           int64_t{kQ * 4} * c->nbk * cand_count_queries(0, c->num_cus);
     const int64_t budget = std::max<int64_t>(int64_t{1} << 30, std::min<int64_t>(int64_t{64} << 30,
-                                                                                 static_cast<int64_t>(free_b / 2)));
+                                                                                 static_cast<int64_t>(free_b / 2))) -
+                           beside;
     int qs = static_cast<int>(std::max<int64_t>(8, std::min<int64_t>(budget / std::max<int64_t>(per_query, 1), 4096)));
     qs = qs / 8 * 8;
-    const int maxb8 = (max_batch + 7) / 8 * 8;
     c->qs = std::min(qs, maxb8);
     c->qs_cap = c->qs;
 
     const WorkspaceShape sh{static_cast<size_t>(max_batch), static_cast<size_t>(c->qs), static_cast<size_t>(c->dim),
                             static_cast<size_t>(opt->nprobe), static_cast<size_t>(c->nbk), static_cast<size_t>(c->vcap),
                             static_cast<size_t>(opt->k_refine), static_cast<size_t>(c->fb_cap), true,
-                            static_cast<size_t>(std::min(c->qs, kSelectSplitQueries)), c->blog};
+                            static_cast<size_t>(cand_count_queries(c->qs, c->num_cus)),
+                            static_cast<size_t>(std::min(c->qs, split)), c->blog};
     unsigned char* block = nullptr;
     // its size varies with the cluster sizes from build to build; it comes
     // last, so a quarter left over takes no room from anything
@@ -1420,7 +1426,7 @@ int chimera_search_device_noalloc(chimera_ctx* c, const float* d_queries, int32_
     const WorkspaceShape sh{static_cast<size_t>(nq), qs, static_cast<size_t>(c->dim),
                             static_cast<size_t>(c->opt.nprobe), static_cast<size_t>(c->nbk),
                             static_cast<size_t>(c->vcap), static_cast<size_t>(c->opt.k_refine),
-                            static_cast<size_t>(c->fb_cap), false, 0, c->blog};
+                            static_cast<size_t>(c->fb_cap), false, qs, 0, c->blog};
     const size_t need = carve_workspace(sh, nullptr, nullptr);
     if (need > kStaticScratchBytes) {
         // the largest batch that fits, for the message
@@ -1429,6 +1435,7 @@ int chimera_search_device_noalloc(chimera_ctx* c, const float* d_queries, int32_
             WorkspaceShape t = sh;
             t.batch = static_cast<size_t>(b);
             t.qs = static_cast<size_t>(std::min(b, c->qs));
+            t.counts = t.qs;
             if (carve_workspace(t, nullptr, nullptr) > kStaticScratchBytes) break;
             fit = b;
         }

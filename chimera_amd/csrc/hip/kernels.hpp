@@ -142,8 +142,12 @@ struct CandidateArgs {
 constexpr int kSelectBins = 4096;
 constexpr int kSelectWords = kSelectBins + 32;
 constexpr int kSelectSplitQueries = 1024;
-constexpr int kCountQueries = 256;  // visit counts are held for at least so many queries
 constexpr int64_t kSelectSplitDocs = 8'000'000;
+// Queries that the split selection can be taken for at num_docs documents.
+int select_split_queries(int64_t num_docs);
+// Queries of visit counts that sub-batches of up to qs queries can use: a
+// small one splits each query's visits over several.
+int cand_count_queries(int qs, int num_cus);
 int cand_buckets(int64_t num_docs, int blog);
 // Bucket size (log2) of the candidate stage for an index: the largest in
 // [kMinBucketLog2, kMaxBucketLog2] at which a (query, bucket) item expects at

@@ -1572,6 +1572,15 @@ int cand_parts(int qs, int num_cus, int wqs) {
     return p;
 }
 
+int cand_count_queries(int qs, int num_cus) {
+    // qs * parts is at most twice the num_cus / kQ that still allow doubling
+    return std::max(qs, 2 * (num_cus / kQ));
+}
+
+int select_split_queries(int64_t num_docs) {
+    return static_cast<int>(std::min<int64_t>(kSelectSplitQueries, kSelectSplitDocs / std::max<int64_t>(num_docs, 1)));
+}
+
 // Segments per query of the visit-count scan: one block per query while the
 // sub-batch fills a quarter of the CUs, else up to 64 segments of at least
 // 256 uint4 each, so that the sub-batch takes about one block per CU (their

@@ -42,6 +42,7 @@ std::map<const void*, std::string> g_names;
 std::map<const void*, std::pair<size_t, void*>> g_vars;
 std::map<std::string, int> g_launches;
 int g_lane_cap = -1;
+std::vector<size_t> g_sizes;  // of every successful hipMalloc, in order
 
 struct Config {
     dim3 grid, block;
@@ -110,6 +111,8 @@ void host_hip_refuse_pointer(int n) { g_refuse_pointer = n; }  // the next n hip
 size_t host_hip_used(void) { return g_used; }
 size_t host_hip_peak(void) { return g_peak; }
 void host_hip_reset_peak(void) { g_peak = g_used; }
+// bytes asked for by the hipMalloc call `back` calls before the last
+size_t host_hip_malloc(int back) { return g_sizes[g_sizes.size() - 1 - static_cast<size_t>(back)]; }
 // launches of kernels whose name holds `part`
 int host_hip_launches(const char* part) {
     Lock lock(g_mu);
@@ -198,6 +201,7 @@ hipError_t hipMalloc(void** p, size_t n) {
     *p = map_bytes(bytes);
     if (!*p) return done(hipErrorOutOfMemory);
     g_blocks[*p] = bytes;
+    g_sizes.push_back(n);
     g_used += bytes;
     if (g_used > g_peak) g_peak = g_used;
     return hipSuccess;

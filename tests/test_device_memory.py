@@ -15,7 +15,7 @@ PRELUDE = """
 import ctypes as C, sys
 import numpy as np
 hip = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)  # before the library, which takes it for its runtime
-for name in ("used", "peak"):
+for name in ("used", "peak", "malloc"):
     getattr(hip, "host_hip_" + name).restype = C.c_size_t
 from chimera_amd import capi
 
@@ -34,6 +34,12 @@ def build(ctx, docs, doc_len=100, clusters=2048, ex_bits=1):
         C.c_uint64(clusters), C.c_uint64(ex_bits), capi._ptr(ids), capi._ptr(flips), C.byref(ctx.options),
         ctx.max_batch))
     ctx._set_shape(n, 128, clusters, ex_bits, lens)
+
+def workspace():
+    \"\"\"Bytes of the last index's search workspace: the last block but the
+    status word's.\"\"\"
+    assert hip.host_hip_malloc(0) == 4
+    return hip.host_hip_malloc(1)
 
 def zeros(nq):
     return np.zeros((nq, 32, 128), np.float32)
@@ -215,4 +221,51 @@ def test_assignment_lists_hold_256_candidates(host_hip):
 ctx = context()
 build(ctx, 20_000)
 assert hip.host_hip_lane_cap() == 256
+""")
+
+
+def test_a_one_query_workspace_holds_the_visit_counts_it_can_use(host_hip):
+    """Visit counts are held for the queries and for the parts that a small
+    batch's visits are split into (16 of them on 256 CUs), not for more."""
+    host_hip("""
+capacity(1 << 40)
+sizes = []
+for batch in (8, 16):
+    ctx = context(max_batch=batch)
+    build(ctx, 10_000_000, doc_len=1, clusters=200_000)
+    sizes.append(workspace())
+    ctx.close()
+assert sizes[0] < 0.56 * sizes[1], sizes
+""")
+
+
+def test_the_split_selection_holds_state_for_the_queries_that_take_it(host_hip):
+    """At 2M documents that is 4 queries. Past k_refine 2048 its lists double
+    (32 KB a query); nothing else grows by more than a word a query."""
+    host_hip("""
+capacity(1 << 40)
+sizes = []
+for k_refine in (2048, 2049):
+    ctx = context(max_batch=1024, k_refine=k_refine)
+    build(ctx, 2_000_000, doc_len=1, clusters=200_000)
+    sizes.append(workspace())
+    ctx.close()
+assert 0 < sizes[1] - sizes[0] < 1 << 20, sizes
+""")
+
+
+def test_the_workspace_stays_within_its_budget(host_hip):
+    """Per-query state, visit counts and split selection together take at most
+    half of the free memory (and at least 1 GiB of budget)."""
+    host_hip("""
+capacity(4500 << 20)
+for k_refine in (60, 4097):
+    ctx = context(max_batch=1024, k_refine=k_refine)
+    build(ctx, 7000, doc_len=300)
+    batch_arrays = 1024 * (32 * (128 * 8 + 8 * 4 + 8) + 65536 + 3 * 4 * k_refine + 512)
+    assert workspace() < (1 << 30) + batch_arrays + (64 << 10), (workspace(), batch_arrays)
+    hip.host_hip_reset_launches()
+    ctx.search(zeros(1024), 10)
+    assert hip.host_hip_launches(b"cand_count") > 1  # the budget bounds the sub-batches
+    ctx.close()
 """)
