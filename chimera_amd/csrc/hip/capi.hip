@@ -550,19 +550,6 @@ hipError_t launch_gather_token_order(hipStream_t s, const uint8_t* codes_clu, co
     return hipGetLastError();
 }
 
-__global__ void copy_u32_kernel(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src, int64_t n) {
-    for (int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; t < n;
-         t += static_cast<int64_t>(gridDim.x) * blockDim.x)
-        dst[t] = src[t];
-}
-
-hipError_t launch_copy_u32(hipStream_t s, uint32_t* dst, const uint32_t* src, int64_t n) {
-    if (n <= 0) return hipSuccess;
-    const int64_t blocks = std::min<int64_t>((n + 255) / 256, 4096);
-    hipLaunchKernelGGL(copy_u32_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, dst, src, n);
-    return hipGetLastError();
-}
-
 hipError_t launch_fill_u32(hipStream_t s, uint32_t* p, int64_t n, uint32_t v) {
     if (n <= 0) return hipSuccess;
     const int64_t blocks = std::min<int64_t>((n + 255) / 256, 4096);

@@ -2,8 +2,6 @@
 // (include/chimera_workload.h).
 #include "capi_internal.hpp"
 #include "chimera_workload.h"
-#include <algorithm>
-
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -347,59 +345,59 @@ __global__ __launch_bounds__(kRescoreWaves * kWave) void maxsim_rescore_kernel(
     }
 }
 
-// The same scores for few candidates: `split` waves of the block share a
-// document (tile t of it goes to wave t mod split), so that its tiles are
-// loaded side by side; their maxima meet in LDS. What bounds a small call is
-// the round trip per tile of the longest document: one query of 100
-// candidates of up to 256 tokens took 57 us with a wave per document, 11 with eight.
+// The same scores for few candidates: the waves of a block (eight or four)
+// share one document, tile t of it going to wave t mod their number, so that
+// its tiles are loaded side by side; their maxima meet in LDS. What bounds a
+// small call is the round trip per tile of the longest document: one query of
+// 100 candidates of up to 256 tokens took 57 us with a wave per document, 11
+// with eight.
 constexpr int kRescoreSmallWaves = 8;
 __global__ __launch_bounds__(kRescoreSmallWaves * kWave) void maxsim_rescore_small_kernel(
     const float* __restrict__ emb, const int32_t* __restrict__ doc_ptrs, int64_t m, const float* __restrict__ queries,
-    const int32_t* __restrict__ cand_ids, const int32_t* __restrict__ cand_counts, int cap, int split,
+    const int32_t* __restrict__ cand_ids, const int32_t* __restrict__ cand_counts, int cap,
     float* __restrict__ scores) {
     __shared__ float part[kRescoreSmallWaves][2][kWave];
     const int q = blockIdx.y;
+    const int j = blockIdx.x;
     const int cnt = cand_counts[q];
     const int n = cnt < 0 ? 0 : (cnt < cap ? cnt : cap);
-    const int per = static_cast<int>(blockDim.x) / kWave / split;
-    if (static_cast<int>(blockIdx.x) * per >= n) return;
+    if (j >= n) return;
     const int l = lane_id();
     const int w = wave_id();
+    const int waves = static_cast<int>(blockDim.x) / kWave;
     const int c = l & 15;
     const int g = l >> 4;
-    const int j = static_cast<int>(blockIdx.x) * per + w / split;
-    const int32_t d = j < n ? cand_ids[static_cast<size_t>(q) * cap + j] : -1;
+    const int32_t d = cand_ids[static_cast<size_t>(q) * cap + j];
     // waves past the document's tiles only meet at the barrier
     const bool in = d >= 0 && d < m;
     const int start = in ? doc_ptrs[d] : 0, end = in ? doc_ptrs[d + 1] : 0;
-    const int mine = w % split;
     float inv[2] = {0.0f, 0.0f};
     float mx0 = -INFINITY, mx1 = -INFINITY;
-    if (start + 16 * mine < end) {
+    if (start + 16 * w < end) {
         half8_t bq[4][2][2];
         load_query_split(queries + static_cast<size_t>(q) * kQ * kDim, c, g, bq, inv);
-        doc_maxsim_tiles(emb, start, end, 16 * mine, 16 * split, bq, c, g, mx0, mx1);
+        doc_maxsim_tiles(emb, start, end, 16 * w, 16 * waves, bq, c, g, mx0, mx1);
     }
     part[w][0][l] = mx0;
     part[w][1][l] = mx1;
     __syncthreads();
-    if (mine != 0 || j >= n) return;
-    for (int o = 1; o < split; ++o) {
-        mx0 = fmaxf(mx0, part[w + o][0][l]);
-        mx1 = fmaxf(mx1, part[w + o][1][l]);
+    if (w != 0) return;
+    for (int o = 1; o < waves; ++o) {
+        mx0 = fmaxf(mx0, part[o][0][l]);
+        mx1 = fmaxf(mx1, part[o][1][l]);
     }
     const float v = start < end ? maxsim_finish(mx0, mx1, inv) : -INFINITY;
     if (l == 0) scores[static_cast<size_t>(q) * cap + j] = v;
 }
 
 // Calls of up to this many candidate documents share each document between
-// waves: eight while that is at most 16 waves a CU, else four. Whole calls
-// with documents of up to 256 tokens: 100 candidates 72 -> 28 us, 900 95 ->
-// 43, 1,800 95 -> 57; of up to 32 tokens: 33 -> 24, 33 -> 30, 34.5 -> 34.6.
-// Past 2,048 the short ones lose (3,000: 36 -> 39 us), as every block loads
-// its query.
+// waves: eight while that is at most 16 waves for each of 256 CUs, else four.
+// Whole calls with documents of up to 256 tokens: 100 candidates 72 -> 28 us,
+// 900 95 -> 43, 1,800 95 -> 57; of up to 32 tokens: 33 -> 24, 33 -> 30, 34.5
+// -> 34.6. Past 2,048 the short ones lose (3,000: 36 -> 39 us), as every
+// block loads its query.
 constexpr int64_t kRescoreSmallDocs = 2048;
-int rescore_split(int64_t docs) { return docs <= 512 ? 8 : 4; }
+int rescore_waves(int64_t docs) { return docs <= 512 ? kRescoreSmallWaves : 4; }
 
 // Matrix-core throughput with register operands: every wave runs `iters`
 // rounds of independent accumulation chains of one instruction type on
@@ -573,11 +571,9 @@ int chimera_maxsim_rescore_device(chimera_ctx* ctx, const float* d_embeddings, c
     stage_begin(ctx, kStageRescore);
     const int64_t docs = static_cast<int64_t>(nq) * cand_cap;
     if (docs <= kRescoreSmallDocs) {
-        const int split = rescore_split(docs);
-        const int waves = std::max(split, 4);
-        const int per = waves / split;
-        hipLaunchKernelGGL(maxsim_rescore_small_kernel, dim3((cand_cap + per - 1) / per, nq), dim3(waves * kWave), 0, s, d_embeddings, d_doc_ptrs, num_docs, d_queries,
-                           d_cand_ids, d_cand_counts, cand_cap, split, d_cand_scores);
+        hipLaunchKernelGGL(maxsim_rescore_small_kernel, dim3(cand_cap, nq), dim3(rescore_waves(docs) * kWave), 0, s,
+                           d_embeddings, d_doc_ptrs, num_docs, d_queries, d_cand_ids, d_cand_counts, cand_cap,
+                           d_cand_scores);
     } else {
         const dim3 grid(static_cast<unsigned>((cand_cap + kRescoreDocsPerBlock - 1) / kRescoreDocsPerBlock),
                         static_cast<unsigned>(nq));

@@ -143,7 +143,7 @@ assert plan(fresh)[0] == other[0]
 
 
 @pytest.mark.parametrize("refuse", ["host_hip_refuse_malloc(C.c_size_t(4 * ctx.n), C.c_size_t(4 * ctx.n))",
-                                    "host_hip_refuse_host(1)"])
+                                    "host_hip_refuse_host(1)"], ids=["positions", "ring"])
 def test_a_download_that_falls_back_leaves_no_error(host_hip, refuse):
     """Without room for the token positions, or without pinned memory, the
     download takes another way; the error it met is not the next call's."""
