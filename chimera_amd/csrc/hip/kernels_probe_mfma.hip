@@ -54,7 +54,10 @@ constexpr int kTileBytes = 32 * kDim * 2;      // 32 centroid rows of 256 B, chu
 constexpr int kWaitVmcnt0 = 0x0F70;            // s_waitcnt vmcnt(0), expcnt and lgkmcnt not waited on
 constexpr int kProbeLaneCap = 128;             // sub-list entries per (row, split, lane half) of the probe
 constexpr int kProbeMaxCandidates = 2048;      // candidates per row the rerank sorts in LDS
-constexpr int kTop1LaneCap = 256;              // sub-list entries of the top-1 search (repeated tokens fill them)
+// Sub-list entries of the top-1 search. Repeated tokens fill them, and rows
+// past them go to the exact kernels: 800,000 tokens over 16,384 clusters, 300
+// of these equal, build in 19 ms with 256 entries and took 118 with 128.
+constexpr int kTop1LaneCap = 256;
 constexpr int kMaxSublists = 1024;             // 2 * splits
 constexpr int64_t kMaxGroups = 16384;          // sampled group minima per row of the probe
 

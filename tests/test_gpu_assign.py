@@ -43,7 +43,7 @@ def test_many_equal_centroids(chimera_mod, repeats):
     rng = np.random.default_rng(repeats)
     x = rng.standard_normal((n, dim)).astype(np.float32)
     ids = np.asarray(chimera_mod._sample_centroid_ids(n, k), np.int64)
-    near = rng.permutation(n)[: n // 2]
+    near = np.setdiff1d(rng.permutation(n)[: n // 2], ids)
     x[near] = x[0] + np.float32(1e-2) * rng.standard_normal((near.size, dim)).astype(np.float32)
     x[ids[rng.permutation(k)[:repeats]]] = x[0]
     lens = np.full(n // 20, 20, np.int32)
