@@ -109,7 +109,7 @@ struct WorkspaceShape {
     size_t batch, qs, dim, nprobe, nbk, vcap, k_refine, fb_cap;
     bool staging;  // query staging and result counts of the host entry points
     size_t counts;  // queries of visit counts
-    size_t split;  // queries of the split selection's state (0: none)
+    size_t split;  // queries of the split selection's state (0: never taken)
     int blog;      // documents per candidate bucket = 2^blog
 };
 
@@ -156,6 +156,8 @@ size_t carve_workspace(const WorkspaceShape& sh, unsigned char* base, Workspace*
     take(x.gsec, QS * sh.nbk * static_cast<size_t>(groups_per_bucket(sh.blog)));
     take(x.gkey, QS * sh.nbk * static_cast<size_t>(groups_per_bucket(sh.blog)));
     take(x.ccount, QS);
+    x.sel = nullptr;
+    x.sel_lists = nullptr;
     if (sh.split > 0) {
         take(x.sel, sh.split * kSelectWords);
         take(x.sel_lists, sh.split * static_cast<size_t>(select_list_cap(static_cast<int>(sh.k_refine))));
@@ -982,7 +984,7 @@ int finish_setup(chimera_ctx* c, const chimera_search_options& o, int32_t max_ba
     // (less what is held beside it: the split selection's state and the visit
     // counts past the sub-batch's)
     const int maxb8 = (max_batch + 7) / 8 * 8;
-    const int split = std::min(maxb8, select_split_queries(c->num_docs));
+    const int split = std::min(maxb8, select_split_queries(c->num_docs, c->blog, opt->k_refine, c->num_cus));
     const int64_t beside = static_cast<int64_t>(split) * (kSelectWords * 4 + int64_t{8} * select_list_cap(opt->k_refine)) +
                            int64_t{kQ * 4} * c->nbk * cand_count_queries(0, c->num_cus);
     const int64_t budget = std::max<int64_t>(int64_t{1} << 30, std::min<int64_t>(int64_t{64} << 30,

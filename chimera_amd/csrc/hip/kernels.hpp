@@ -136,15 +136,12 @@ struct CandidateArgs {
     uint64_t* sel_lists;  // [sel_queries][select_list_cap(k_refine)]
     int sel_queries;
 };
-// Split selection: histogram bins, words of state per query (a multiple of
-// the 32 tokens), the most queries it holds state for, and the most documents
-// times queries of a sub-batch.
+// Split selection: histogram bins, and words of state per query (a multiple of
+// the 32 tokens).
 constexpr int kSelectBins = 4096;
 constexpr int kSelectWords = kSelectBins + 32;
-constexpr int kSelectSplitQueries = 1024;
-constexpr int64_t kSelectSplitDocs = 8'000'000;
-// Queries that the split selection can be taken for at num_docs documents.
-int select_split_queries(int64_t num_docs);
+// The most queries of a sub-batch that takes the split selection (0: none).
+int select_split_queries(int64_t num_docs, int blog, int k_refine, int num_cus);
 // Queries of visit counts that sub-batches of up to qs queries can use: a
 // small one splits each query's visits over several.
 int cand_count_queries(int qs, int num_cus);

@@ -1577,10 +1577,6 @@ int cand_count_queries(int qs, int num_cus) {
     return std::max(qs, 2 * (num_cus / kQ));
 }
 
-int select_split_queries(int64_t num_docs) {
-    return static_cast<int>(std::min<int64_t>(kSelectSplitQueries, kSelectSplitDocs / std::max<int64_t>(num_docs, 1)));
-}
-
 // Segments per query of the visit-count scan: one block per query while the
 // sub-batch fills a quarter of the CUs, else up to 64 segments of at least
 // 256 uint4 each, so that the sub-batch takes about one block per CU (their
@@ -1600,18 +1596,32 @@ static int log2_of(int p) {
     return l;
 }
 
-// Whether a sub-batch of qs queries takes the split selection: its candidates
-// (at most a document each, read three times) are few enough, and either the
-// groups cannot prune (fewer than 4 k_refine of them, so the query-per-block
-// kernel walks every candidate) or it leaves half of the CUs idle. A search
-// of 52 queries over 150,000 documents (7.8M documents times queries, groups
-// that do not prune): 1,736 us without, 1,466 with; 26 over 300,000: 1,010
-// and 975; 300 over 150,000 (45M): 7,331 and 7,531.
-static bool select_split(const CandidateArgs& a, int qs) {
-    if (a.sel == nullptr || qs > a.sel_queries || static_cast<int64_t>(qs) * a.num_docs > kSelectSplitDocs) return false;
-    const int64_t groups = static_cast<int64_t>(a.nbk) * groups_per_bucket(a.blog);
-    return groups < 4 * static_cast<int64_t>(a.k_refine) || qs <= a.num_cus / 2;
+// When a sub-batch takes the split selection. It reads every candidate (at
+// most a document each) three times, which costs 6-10 us per million
+// documents times queries. What it saves depends on whether the
+// query-per-block kernel can prune by the maxima of the document groups:
+//   groups <= k_refine: it cannot, and walks every candidate with one block
+//     a query. Whole searches before and after, us: 150,000 documents
+//     (k_refine 3000), 26 queries 921 and 709, 52 1,372 and 1,184; 100,000
+//     (1500), 8 435 and 310, 80 1,531 and 1,398; 40,000 (1000), 100 881 and
+//     836, 200 1,555 and 1,548, 300 2,236 and 2,274. Past a query per CU the
+//     blocks fill the GPU: 10,000 (1000), 400 queries 1,939 and 1,954.
+//   else it lists a few candidates more than k_refine. Its sort grows with
+//     the list: past k_refine 2048 one query over 250,000 documents (3000)
+//     takes 262 and 227, 13 496 and 477, 26 752 and 753; 300,000 (3000), 13
+//     487 and 473, 26 678 and 686; 1M (3000), 4 319 and 315, 8 419 and 428.
+//     From 1024 to 2048: 300,000 (2000), one 215 and 205, 4 263 and 258, 13
+//     431 and 441; 150,000 (1500), 6 294 and 287, 26 602 and 614. Up to 1024
+//     nothing is saved: 150,000 (1000), 6 271 and 274, 52 887 and 939;
+//     20,000 (200), 25 246 and 252, 200 725 and 765.
+int select_split_queries(int64_t num_docs, int blog, int k_refine, int num_cus) {
+    const int64_t groups = static_cast<int64_t>(cand_buckets(num_docs, blog)) * groups_per_bucket(blog);
+    const int64_t docs = std::max<int64_t>(num_docs, 1);  // of all queries
+    if (groups <= k_refine) return static_cast<int>(std::min<int64_t>(num_cus, 8'000'000 / docs));
+    return static_cast<int>((k_refine > 2048 ? 4'000'000 : k_refine > 1024 ? 1'000'000 : 0) / docs);
 }
+
+static bool select_split(const CandidateArgs& a, int qs) { return a.sel != nullptr && qs <= a.sel_queries; }
 
 template <int kBlog>
 static void launch_select(hipStream_t s, const CandidateArgs& a, int bshift, int q_base, int qs, int cap) {

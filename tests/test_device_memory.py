@@ -240,8 +240,8 @@ assert sizes[0] < 0.56 * sizes[1], sizes
 
 
 def test_the_split_selection_holds_state_for_the_queries_that_take_it(host_hip):
-    """At 2M documents that is 4 queries. Past k_refine 2048 its lists double
-    (32 KB a query); nothing else grows by more than a word a query."""
+    """At 2M documents that is 2 queries at most. Past k_refine 2048 its lists
+    double (32 KB a query); nothing else grows by more than a word a query."""
     host_hip("""
 capacity(1 << 40)
 sizes = []
@@ -268,4 +268,25 @@ for k_refine in (60, 4097):
     ctx.search(zeros(1024), 10)
     assert hip.host_hip_launches(b"cand_count") > 1  # the budget bounds the sub-batches
     ctx.close()
+""")
+
+
+# documents, k_refine, queries of the batch, split: on either side of every
+# line of the rule (64 documents a group)
+@pytest.mark.parametrize("docs,k_refine,nq,split", [
+    (50_000, 1000, 160, True), (50_000, 1000, 161, False),    # the groups cannot prune: 8M documents of all queries
+    (10_000, 1000, 256, True), (10_000, 1000, 257, False),    # and a query a CU
+    (200_000, 2500, 20, True), (200_000, 2500, 21, False),    # more groups, lists past 4,096 keys: 4M
+    (100_000, 1500, 10, True), (100_000, 1500, 11, False),    # shorter lists: 1M
+    (100_000, 1024, 1, False), (20_000, 200, 1, False),       # short lists
+    (5_000_000, 3000, 1, False)])
+def test_calls_that_take_the_split_selection(host_hip, docs, k_refine, nq, split):
+    host_hip(f"""
+capacity(1 << 40)
+ctx = context(max_batch=300, k_refine={k_refine})
+build(ctx, {docs}, doc_len=1, clusters=4096)
+hip.host_hip_reset_launches()
+ctx.search(zeros({nq}), 10)
+assert hip.host_hip_launches(b"select_refine") == 1
+assert hip.host_hip_launches(b"select_collect") == {int(split)}
 """)

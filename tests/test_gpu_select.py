@@ -47,3 +47,11 @@ def test_refined_lists(chimera_mod, docs, clusters, nprobe, k_refine, scale, cop
         assert np.array_equal(t["refined_ids"][q, :n], ref["refined_ids"])
         if q == 0:
             assert np.array_equal(one["refined_ids"][0, :n], ref["refined_ids"])
+
+
+# further shapes that take it: larger buckets whose groups cannot prune, and
+# more groups than k_refine with lists of 4,096 and of 8,192 keys
+@pytest.mark.parametrize("docs,clusters,nprobe,k_refine", [(30000, 4096, 24, 500), (80000, 64, 24, 1100),
+                                                           (150000, 64, 24, 2100)])
+def test_refined_lists_of_more_documents(chimera_mod, docs, clusters, nprobe, k_refine):
+    test_refined_lists(chimera_mod, docs, clusters, nprobe, k_refine, 1.0, 0)
