@@ -722,11 +722,12 @@ hipError_t launch_encode_tokens(hipStream_t s, const float* emb, int64_t n, int 
         hipLaunchKernelGGL(kernel, dim3(grid), dim3(kEncWaves * kWave), 0, s, emb, n, dim, flips, fac, ex_bits, codes1, f1,
                            full, fF, status);
     };
-    // more intervals leave fewer events to step through, which pays from
-    // 7-bit codes on: 2.9M tokens at ex_bits 7 25.1 ms with 512 and 28.9 with
-    // 256, 0.88M at ex_bits 4 3.9 and 3.5 ms (before the
-    // dimensions were sorted for the walk)
-    if (ex_bits >= 6)
+    // More intervals leave fewer events to step through and cost a longer
+    // scan and a wave less per SIMD, which pays at 8-bit codes only. 2.9M
+    // tokens with 256 and with 512, ms, by ex_bits: 4 9.68 and 11.10, 5 10.73
+    // and 11.88, 6 15.04 and 15.17, 7 26.92 and 23.06; of 96 dimensions 6
+    // 14.29 and 14.43, 7 26.14 and 22.12.
+    if (ex_bits >= 7)
         encode(encode_tokens_kernel<512>);
     else
         encode(encode_tokens_kernel<256>);

@@ -290,3 +290,11 @@ ctx.search(zeros({nq}), 10)
 assert hip.host_hip_launches(b"select_refine") == 1
 assert hip.host_hip_launches(b"select_collect") == {int(split)}
 """)
+
+
+@pytest.mark.parametrize("ex_bits,intervals", [(1, 256), (6, 256), (7, 512)])
+def test_the_encoders_intervals(host_hip, ex_bits, intervals):
+    host_hip(f"""
+build(context(), 1000, ex_bits={ex_bits})
+assert hip.host_hip_launches(b"encode_tokens_kernelILi{intervals}E") == 1
+""")
