@@ -14,7 +14,22 @@ namespace chimera {
 
 namespace {
 
-__constant__ float kTightStart[9] = {0.F, 0.15F, 0.20F, 0.52F, 0.59F, 0.71F, 0.75F, 0.77F, 0.81F};
+struct TightStart {
+    float of[9];  // by ex_bits
+};
+constexpr TightStart kTightStartValues = {{0.F, 0.15F, 0.20F, 0.52F, 0.59F, 0.71F, 0.75F, 0.77F, 0.81F}};
+__constant__ TightStart kTightStart = kTightStartValues;
+
+// The rescale search's range of t in units of 1 / max |o|, the least spacing
+// of one dimension's events.
+constexpr double rescale_spacings(int ex_bits) {
+    return ((1 << ex_bits) + 9) * (1.0 - static_cast<double>(kTightStartValues.of[ex_bits]));
+}
+constexpr double most_rescale_spacings() {
+    double most = 0.0;
+    for (int e = 1; e <= 7; ++e) most = rescale_spacings(e) > most ? rescale_spacings(e) : most;
+    return most;
+}
 
 __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
     const uint32_t lo = __shfl_xor(static_cast<uint32_t>(v), m, kWave);
@@ -257,8 +272,8 @@ __device__ double rescale_sequential(const RescaleLane& in, const float* sabs, d
 // 53 bits.
 //
 // An interval is narrower than 1 / max a = the least spacing of one
-// dimension's events (the range is at most 26 spacings for every ex_bits), so
-// a dimension has at most one event in it.
+// dimension's events (the range is at most 31.5 spacings, at ex_bits 7), so a
+// dimension has at most one event in it.
 //
 // The walk takes as many steps as the lane with the most events, so its lanes
 // do not take the dimensions that they own: the dimensions are sorted by event
@@ -266,7 +281,7 @@ __device__ double rescale_sequential(const RescaleLane& in, const float* sabs, d
 // from either end. On Gaussian tokens at ex_bits 7 that is 28 steps instead
 // of 42 (11 to 7.5 at ex_bits 4): 2.9M tokens 25.2 -> 23.8 ms, 0.88M at
 // ex_bits 4 3.56 -> 3.51 ms.
-constexpr int kOrderKeys = 32;
+constexpr int kOrderKeys = 32;  // counts past 31 (of at most 33) share a key: the order only evens out the walk
 template <int kBins>
 union RescaleBins {
     struct {
@@ -284,6 +299,7 @@ union RescaleBins {
 template <int kBins>
 __device__ double rescale_binned(const RescaleLane& in, RescaleBins<kBins>& bins, double t_start, double t_end, double num0,
                                  double den0, int top, int l) {
+    static_assert(2.0 * most_rescale_spacings() < kBins, "at most one event of a dimension in an interval");
     constexpr int kPerLane = kBins / kWave;
     const double ya = in.oa > 0.0f ? 1.0 / static_cast<double>(in.oa) : 0.0;
     const double yb = in.ob > 0.0f ? 1.0 / static_cast<double>(in.ob) : 0.0;
@@ -584,7 +600,7 @@ __global__ __launch_bounds__(kEncWaves * kWave, kBins <= 256 ? 4 : 3) void encod
             }
             if (l == 0) sbad[i] = 0u;
             const double t_end = static_cast<double>(top + 10) / static_cast<double>(max_o);
-            const double t_start = t_end * static_cast<double>(kTightStart[ex_bits]);
+            const double t_start = t_end * static_cast<double>(kTightStart.of[ex_bits]);
             in.ca = static_cast<int>(fma(t_start, static_cast<double>(in.oa), 1e-5));
             in.cb = static_cast<int>(fma(t_start, static_cast<double>(in.ob), 1e-5));
             const double den = static_cast<double>(kDim) * 0.25 +
