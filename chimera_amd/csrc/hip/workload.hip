@@ -345,13 +345,13 @@ __global__ __launch_bounds__(kRescoreWaves * kWave) void maxsim_rescore_kernel(
     }
 }
 
-// The same scores for few candidates: the waves of a block (eight or four)
+// The same scores for few candidates: the waves of a block (four or two)
 // share one document, tile t of it going to wave t mod their number, so that
 // its tiles are loaded side by side; their maxima meet in LDS. What bounds a
 // small call is the round trip per tile of the longest document: one query of
-// 100 candidates of up to 256 tokens took 57 us with a wave per document, 11
-// with eight.
-constexpr int kRescoreSmallWaves = 8;
+// 100 candidates of up to 256 tokens takes 75 us as a whole call with a wave
+// per document, 27 with four.
+constexpr int kRescoreSmallWaves = 4;
 __global__ __launch_bounds__(kRescoreSmallWaves * kWave) void maxsim_rescore_small_kernel(
     const float* __restrict__ emb, const int32_t* __restrict__ doc_ptrs, int64_t m, const float* __restrict__ queries,
     const int32_t* __restrict__ cand_ids, const int32_t* __restrict__ cand_counts, int cap,
@@ -391,13 +391,23 @@ __global__ __launch_bounds__(kRescoreSmallWaves * kWave) void maxsim_rescore_sma
 }
 
 // Calls of up to this many candidate documents share each document between
-// waves: eight while that is at most 16 waves for each of 256 CUs, else four.
-// Whole calls with documents of up to 256 tokens: 100 candidates 72 -> 28 us,
-// 900 95 -> 43, 1,800 95 -> 57; of up to 32 tokens: 33 -> 24, 33 -> 30, 34.5
-// -> 34.6. Past 2,048 the short ones lose (3,000: 36 -> 39 us), as every
-// block loads its query.
+// waves: four up to 512, else two. Every block loads its query, so more waves
+// than tiles are paid for, most of all with other calls in flight. A whole
+// call alone / with three contexts' calls in flight, us, by waves (one: the
+// kernel above), documents of up to 32 and of up to 256 tokens:
+//     documents        1            2            4            8
+//     400   32 t   32.3 / 8.2   24.5 / 8.3   24.5 / 8.3   26.5 / 8.3
+//          256 t   82.1 / 28.4  33.9 / 9.4   31.8 / 9.3   35.8 / 11.4
+//     1000  32 t   32.6 / 10.0  27.1 / 8.2   29.1 / 8.6   32.7 / 14.1
+//          256 t   94.9 / 32.3  38.9 / 15.1  42.8 / 17.7  51.7 / 27.2
+//     1564  32 t   32.6 / 10.3  30.1 / 10.3  31.9 / 12.6  41.8 / 22.3
+//          256 t   94.1 / 39.4  48.2 / 26.8  51.9 / 30.2  67.6 / 44.2
+//     2000  32 t   33.8 / 10.7  32.8 / 12.3  35.0 / 15.1  47.2 / 28.0
+//          256 t   95.3 / 40.8  53.5 / 33.4  57.8 / 37.5  78.8 / 55.5
+//     4000  32 t   40.9 / 12.6  42.6 / 21.6  48.4 / 28.0  76.6 / 54.7
+//          256 t  121.0 / 53.3  83.0 / 64.0  93.1 / 72.2 136.3 / 109.8
 constexpr int64_t kRescoreSmallDocs = 2048;
-int rescore_waves(int64_t docs) { return docs <= 512 ? kRescoreSmallWaves : 4; }
+int rescore_waves(int64_t docs) { return docs <= 512 ? kRescoreSmallWaves : 2; }
 
 // Matrix-core throughput with register operands: every wave runs `iters`
 // rounds of independent accumulation chains of one instruction type on

@@ -41,6 +41,7 @@ thread_local hipError_t g_last = hipSuccess;
 std::map<const void*, std::string> g_names;
 std::map<const void*, std::pair<size_t, void*>> g_vars;
 std::map<std::string, int> g_launches;
+std::map<std::string, int> g_threads;  // of the last launch of each kernel
 int g_lane_cap = -1;
 std::vector<size_t> g_sizes;  // of every successful hipMalloc, in order
 
@@ -124,6 +125,14 @@ int host_hip_launches(const char* part) {
 void host_hip_reset_launches(void) {
     Lock lock(g_mu);
     g_launches.clear();
+    g_threads.clear();
+}
+// threads per block of the last launch of a kernel whose name holds `part` (0: none)
+int host_hip_threads(const char* part) {
+    Lock lock(g_mu);
+    for (const auto& l : g_threads)
+        if (l.first.find(part) != std::string::npos) return l.second;
+    return 0;
 }
 // candidates per sub-list in the last launch of the assignment's rerank (its argument 6)
 int host_hip_lane_cap(void) { return g_lane_cap; }
@@ -161,6 +170,7 @@ hipError_t hipLaunchKernel(const void* function, dim3 grid, dim3 block, void** a
         return done(hipErrorInvalidConfiguration);
     const std::string& name = g_names[function];
     ++g_launches[name];
+    g_threads[name] = static_cast<int>(block.x * block.y * block.z);
     if (name.find("probe_top1_rerank_kernel") != std::string::npos) g_lane_cap = *static_cast<int*>(args[6]);
     push(stream, run(name, args));
     return hipSuccess;

@@ -1,5 +1,5 @@
 """MaxSim rescoring at the sizes where its kernels change (documents shared
-by eight and four waves, a wave per document) and at the edges of the
+by four and two waves, a wave per document) and at the edges of the
 16-token tiles, against float64. Split fp16 operands keep a product within
 2^-21 of |q||x|, so a 32-token sum stays within 32 * 2^-20 of unit vectors'."""
 import numpy as np
