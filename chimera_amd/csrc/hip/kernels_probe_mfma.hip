@@ -809,8 +809,9 @@ __global__ __launch_bounds__(256) void probe_threshold_kernel(const float* __res
 // (kPerLane per lane, for rows of at most 64 kPerLane minima): a binary
 // search on the key's bits, each step a count of the keys below by ballots,
 // ended by the first bound with exactly rank keys below it (about half of
-// the bits). No LDS: four radix passes over LDS histograms took 12.6 us for
-// 32 rows of 1,024 minima and 66 us for 32,768; this XXX.
+// the bits). No LDS and four rows a block: 32,768 rows of 1,024 minima take
+// 54 us against 121 of the radix kernel above. Its chain is longer, though,
+// and with few rows that is all there is to it (threshold_by_waves).
 template <int kPerLane>
 __global__ __launch_bounds__(256) void probe_threshold_wave_kernel(const float* __restrict__ gm, int n_groups,
                                                                    int nrows, int rank, const float* __restrict__ rot,
@@ -1304,6 +1305,21 @@ hipError_t launch_probe_centroids(hipStream_t s, const float* c, const float* no
     return hipGetLastError();
 }
 
+// Which threshold kernel: a wave per row while its registers hold the row's
+// minima and there are rows for all CUs, or the minima are few. Kernel alone,
+// radix and wave, us, by minima and rows:
+//     128    32 rows 5.4 and 5.0, 512 5.9 and 5.6, 8,192 21.5 and 9.6
+//     512    32 6.2 and 7.1, 512 6.5 and 8.2, 2,048 8.8 and 8.4, 8,192 26.9 and 11.9
+//     1,024  32 7.4 and 10.2, 512 7.8 and 11.5, 4,096 19.0 and 14.5
+//     1,563  32 9.5 and 16.3, 512 10.2 and 17.7, 4,096 26.6 and 23.6
+// (256 take the same either way). With other contexts' kernels on the GPU the
+// wave kernel's fewer waves count from about 400 rows on: probes from three
+// contexts over 300,000 centroids, us each, 224 rows 54.4 and 54.9, 300 68.5
+// and 69.1, 512 89.0 and 87.2, 2,048 261 and 257.
+static bool threshold_by_waves(int nrows, int n_groups) {
+    return n_groups <= 32 * kWave && (n_groups <= 256 || nrows > 384);
+}
+
 ProbePlan plan_probe_mfma(int nrows, int64_t k, int nprobe, int num_cus) {
     ProbePlan p{};
     const int64_t ntiles = (k + 31) / 32;
@@ -1401,18 +1417,18 @@ hipError_t launch_probe_mfma(hipStream_t s, const ProbePlan& p, const float* rot
         }
         if ((e = hipGetLastError()) != hipSuccess) return e;
         const dim3 wgrid((nrows + 3) / 4);
-        if (n_groups <= 8 * kWave)
+        if (!threshold_by_waves(nrows, n_groups))
+            hipLaunchKernelGGL(probe_threshold_kernel, dim3(nrows), dim3(256), static_cast<size_t>(n_groups) * 4, s,
+                               gm, n_groups, nrows, p.u_rank, rot, cmax, ec, eqw, thr, row_flag, fb.nflag);
+        else if (n_groups <= 8 * kWave)
             hipLaunchKernelGGL(probe_threshold_wave_kernel<8>, wgrid, dim3(256), 0, s, gm, n_groups, nrows, p.u_rank,
                                rot, cmax, ec, eqw, thr, row_flag, fb.nflag);
         else if (n_groups <= 16 * kWave)
             hipLaunchKernelGGL(probe_threshold_wave_kernel<16>, wgrid, dim3(256), 0, s, gm, n_groups, nrows,
                                p.u_rank, rot, cmax, ec, eqw, thr, row_flag, fb.nflag);
-        else if (n_groups <= 32 * kWave)
+        else
             hipLaunchKernelGGL(probe_threshold_wave_kernel<32>, wgrid, dim3(256), 0, s, gm, n_groups, nrows,
                                p.u_rank, rot, cmax, ec, eqw, thr, row_flag, fb.nflag);
-        else
-            hipLaunchKernelGGL(probe_threshold_kernel, dim3(nrows), dim3(256), static_cast<size_t>(n_groups) * 4, s,
-                               gm, n_groups, nrows, p.u_rank, rot, cmax, ec, eqw, thr, row_flag, fb.nflag);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (part < 0 || part == 1) {

@@ -57,3 +57,24 @@ capi.check(capi.lib().chimera_maxsim_rescore_device(
 assert hip.host_hip_threads(b"maxsim_rescore_small_kernel") == 64 * {waves}
 assert hip.host_hip_launches(b"maxsim_rescore") == 1
 """)
+
+
+def probe_launches(host_hip, clusters, rows, *kernels):
+    host_hip(f"""
+ctx = context(max_batch=128, nprobe=128, k_refine=200)
+build(ctx, 4000, doc_len=100, clusters={clusters})
+hip.host_hip_reset_launches()
+buf = C.c_void_p(4096)
+capi.check(capi.lib().chimera_probe_device(ctx.handle, buf, {rows}, 128, buf))
+for kernel in {kernels}:
+    assert hip.host_hip_launches(kernel.encode()) == 1, kernel
+""")
+
+
+# sampled minima of a row: 128, 256, 257, 1,024, 1,559
+@pytest.mark.parametrize("clusters,rows,kernel", [
+    (4096, 32, "wave_kernelILi8E"), (8192, 32, "wave_kernelILi8E"), (8193, 384, "kernelEPKf"),
+    (8193, 385, "wave_kernelILi8E"), (131_072, 384, "kernelEPKf"), (131_072, 385, "wave_kernelILi16E"),
+    (399_000, 32, "kernelEPKf"), (399_000, 4096, "wave_kernelILi32E")])
+def test_the_threshold_kernel(host_hip, clusters, rows, kernel):
+    probe_launches(host_hip, clusters, rows, "probe_threshold_" + kernel)
