@@ -47,7 +47,8 @@ struct ProbePlan {
     int group_tiles;  // sampled tiles per group minimum of the sampled pass
     int u_rank;       // rank (1-based) of the group minimum that sets the filter threshold
     int lane_cap;  // candidate sub-list entries per (row, split, lane half)
-    int wave_share;  // waves that share 64 rows (1, 2 or 8)
+    int sample_share;  // waves that share 64 rows in the sampled pass (1 or 2)
+    int scan_share;  // and in the filtered pass (1, 2 or 8)
     bool usable;
 };
 // Rows of sub-list storage (buffers hold rows * 2 * lane_cap candidates and

@@ -215,7 +215,7 @@ __global__ __launch_bounds__(256) void probe_centroids_kernel(const float* __res
 // Their hits append to the same sub-lists through counters in LDS (the
 // rerank sorts, so the order of records is free), and the tile minima of a
 // stage meet in LDS. One query over 262,144 centroids: filtered pass 34 -> 22
-// us (3.0 TB/s of centroids), sampled pass 11.7 -> 10.6.
+// us (3.0 TB/s of centroids). plan_probe_mfma says when.
 template <int MODE, int G = kGroupTiles, int TS = 1>
 __global__ __launch_bounds__(kProbeWaves * kWave) void probe_mfma_kernel(
     const float* __restrict__ rot, int nrows, const uint16_t* __restrict__ cbf, const float* __restrict__ nhalf,
@@ -1368,8 +1368,19 @@ ProbePlan plan_probe_mfma(int nrows, int64_t k, int nprobe, int num_cus) {
     p.tiles_per_split = (p.tiles_per_split + unit - 1) / unit * unit;
     p.splits = static_cast<int>((ntiles + p.tiles_per_split - 1) / p.tiles_per_split);
     p.lane_cap = kProbeLaneCap;
-    // one row block that its rows do not fill: waves share the rows there are
-    p.wave_share = nrows <= kRowsPerBlock / 8 ? 8 : nrows <= kRowsPerBlock / 2 ? 2 : 1;
+    // Few rows: waves share them. us with 1, 2 and 8 waves sharing:
+    //   sampled pass and threshold  64 rows 17.3 16.1 18.6 (4,096 centroids),
+    //     22.9 21.7 24.0 (262,144); 128 rows 17.9 17.5 and 23.8 23.4; 256
+    //     19.5 20.6 and 25.5 26.4
+    //   filtered pass  64 rows 12.5 12.4 14.8 (4,096), 24.8 22.2 19.8 (20,000),
+    //     40.3 35.0 27.9 (262,144); 128 13.4 14.0 (4,096), 25.7 24.3 (20,000),
+    //     42.1 37.6 (262,144); 256 15.0 17.8, 27.6 29.7 and 44.8 47.2
+    // and with three contexts' probes on the GPU 256 rows 49 54 (262,144) and
+    // 119 132 (1M) a call. A split of one stage (up to 8,192 centroids) has
+    // each wave take a tile or none, so eight only meet there.
+    const bool one_stage = p.tiles_per_split <= kStageTiles;
+    p.sample_share = nrows <= kRowsPerBlock / 4 ? 2 : 1;
+    p.scan_share = nrows <= kRowsPerBlock / 8 ? (one_stage ? 2 : 8) : nrows <= kRowsPerBlock / 4 && !one_stage ? 2 : 1;
     const int n_groups = (p.n_sampled + p.group_tiles - 1) / p.group_tiles;
     p.usable = n_groups >= nprobe && n_groups <= kMaxGroups && nprobe <= 1024 && 2 * p.splits <= kMaxSublists;
     return p;
@@ -1406,12 +1417,10 @@ hipError_t launch_probe_mfma(hipStream_t s, const ProbePlan& p, const float* rot
                                    p.lane_cap, row_flag, nullptr, cmax, ecmax, p.row_blocks, p.splits);
             };
             if (p.group_tiles == kGroupTiles) {
-                if (p.wave_share == 8) pass(probe_mfma_kernel<0, kGroupTiles, 8>);
-                else if (p.wave_share == 2) pass(probe_mfma_kernel<0, kGroupTiles, 2>);
+                if (p.sample_share == 2) pass(probe_mfma_kernel<0, kGroupTiles, 2>);
                 else pass(probe_mfma_kernel<0, kGroupTiles, 1>);
             } else {
-                if (p.wave_share == 8) pass(probe_mfma_kernel<0, 1, 8>);
-                else if (p.wave_share == 2) pass(probe_mfma_kernel<0, 1, 2>);
+                if (p.sample_share == 2) pass(probe_mfma_kernel<0, 1, 2>);
                 else pass(probe_mfma_kernel<0, 1, 1>);
             }
         }
@@ -1442,8 +1451,8 @@ hipError_t launch_probe_mfma(hipStream_t s, const ProbePlan& p, const float* rot
                                    p.tiles_per_split, 1, gm, thr, nullptr, rv, rtile, cnt, p.lane_cap, row_flag, nullptr,
                                    cmax, ecmax, p.row_blocks, p.splits);
             };
-            if (p.wave_share == 8) pass(probe_mfma_kernel<1, kGroupTiles, 8>);
-            else if (p.wave_share == 2) pass(probe_mfma_kernel<1, kGroupTiles, 2>);
+            if (p.scan_share == 8) pass(probe_mfma_kernel<1, kGroupTiles, 8>);
+            else if (p.scan_share == 2) pass(probe_mfma_kernel<1, kGroupTiles, 2>);
             else pass(probe_mfma_kernel<1, kGroupTiles, 1>);
         }
         if ((e = hipGetLastError()) != hipSuccess) return e;

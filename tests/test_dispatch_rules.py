@@ -78,3 +78,13 @@ for kernel in {kernels}:
     (399_000, 32, "kernelEPKf"), (399_000, 4096, "wave_kernelILi32E")])
 def test_the_threshold_kernel(host_hip, clusters, rows, kernel):
     probe_launches(host_hip, clusters, rows, "probe_threshold_" + kernel)
+
+
+# waves that share 64 rows, in the sampled and in the filtered pass; splits of
+# one stage up to 8,192 centroids
+@pytest.mark.parametrize("clusters,rows,sampled,filtered", [
+    (8192, 32, 2, 2), (8192, 64, 2, 2), (8192, 65, 2, 1), (8192, 128, 2, 1), (8192, 129, 1, 1),
+    (20_000, 64, 2, 8), (20_000, 65, 2, 2), (20_000, 128, 2, 2), (20_000, 129, 1, 1), (262_144, 32, 2, 8)])
+def test_the_waves_that_share_probe_rows(host_hip, clusters, rows, sampled, filtered):
+    probe_launches(host_hip, clusters, rows, f"probe_mfma_kernelILi0ELi1ELi{sampled}E",
+                   f"probe_mfma_kernelILi1ELi4ELi{filtered}E")
